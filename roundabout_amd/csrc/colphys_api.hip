@@ -454,9 +454,19 @@ int staged_coefficients(rdb_colphys* h, int p0, int p1, double dt) {
     // one-pass tail (merge, KV_ML_INVZ2, convection, split, assemble); the
     // KPP overlay needs PP81's values first, so PP81 then stays separate
     // (over every column: a dry column still books its B0)
-    if (h->cfg.epbl_enable)
-      hipLaunchKernelGGL(colphys::k_epbl, grid1(h->n_all - p0, 64), dim3(64), 0, h->stream, h->s, h->ep, h->ev,
-                         h->d_coriolis, h->cfg.rho0, h->cfg.cp, dt, p0, h->n_all);
+    if (h->cfg.epbl_enable) {
+      const colphys::EpblParams& c = h->ep;
+      // the default schemes compile to a kernel without the pow calls and
+      // branches of the others
+      const bool gen = c.mstar_scheme == RDB_EPBL_MSTAR_RH18 || c.vstar_scheme == RDB_EPBL_VSTAR_RH18 || c.use_lt ||
+                       c.mixlen_exponent != 2.0;
+      hipLaunchKernelGGL(gen ? colphys::k_epbl<true> : colphys::k_epbl<false>, grid1(h->n_all - p0, 64), dim3(64), 0,
+                         h->stream, h->s, h->ep, h->ev, h->d_coriolis, h->cfg.rho0, h->cfg.cp, dt, p0, h->n_all);
+      if (c.mld_iteration)
+        hipLaunchKernelGGL(gen ? colphys::k_epbl_bed<true> : colphys::k_epbl_bed<false>,
+                           dim3(std::min(256u, grid1(h->n_all - p0, 64).x)), dim3(512), 0, h->stream, h->s, h->ep,
+                           h->ev, h->d_coriolis, h->cfg.rho0, h->cfg.cp, dt);
+    }
     const int fold_pp81 = h->cfg.use_kpp ? 0 : 1;
     if (!fold_pp81) {
       hipLaunchKernelGGL(colphys::k_pp81, g, b, 0, h->stream, h->s, h->pr, p0, p1);
@@ -812,6 +822,9 @@ int create_plan(const rdb_colphys_config* cfg, int nx, int ny, int nz, int n_pas
     A(&h->ev.b0, 8 * P);
     A(&h->ev.la, 8 * P);
     if (h->cfg.epbl_tke_diags) A(&h->ev.tke, 8 * 6 * P);
+    A(&h->ev.bed_list, sizeof(int) * P);
+    A(&h->ev.bed_count, sizeof(unsigned int));
+    A(&h->ev.bed_done, sizeof(unsigned int));
   }
   h->stage_elems = (size_t)(nx + 1) * (size_t)(ny + 1) * (size_t)(nz + 1);
   A(&h->d_stage, 8 * h->stage_elems);

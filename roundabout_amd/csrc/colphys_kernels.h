@@ -105,14 +105,26 @@ struct EpblParams {
 // mixing, mech_decay, conv_decay), the rest [P].
 struct EpblView {
   double *kd, *mld, *b0, *la, *tke;
+  // columns mixed to the bed that k_epbl leaves to k_epbl_bed, their number,
+  // and the workgroups of k_epbl_bed that have finished (both 0 between solves)
+  int* bed_list;            // [P]
+  unsigned int* bed_count;
+  unsigned int* bed_done;
 };
 // The per-interface contributors after the surface scheme.
 struct ContribParams {
   int epbl, conv, combine, pad;
   double prandtl, kv_ml_invz2, hmix, conv_kd, conv_prandtl, n2_thresh, rho0;
 };
+// GEN = false: OM4 or constant m*, cube-root v*, the mixing-length exponent 2
+// and no Langmuir enhancement; GEN = true: every scheme
+template <bool GEN>
 __global__ void k_epbl(StateView s, EpblParams c, EpblView e, const double* fcor, double rho0, double cp, double dt,
                        int p0, int p1);
+// the columns that k_epbl leaves on e.bed_list, 512 threads a workgroup
+template <bool GEN>
+__global__ void k_epbl_bed(StateView s, EpblParams c, EpblView e, const double* fcor, double rho0, double cp,
+                           double dt);
 __global__ void k_coeff_tail(StateView s, Params pr, ContribParams c, EpblView e, int do_pp81, int p0, int p1,
                              unsigned int* guard_count);
 __global__ void k_safe_math_eval(int fn, const double* x, const double* y, double* out, int n);

@@ -18,8 +18,6 @@
 // each iteration recomputes them on the fly while it walks down (the same
 // pressure stack, summed in the same order, so the same bits): every
 // iteration streams h, T and S only, and no work array is written.
-#include <type_traits>
-
 #include "colphys_kernels.h"
 #include "safe_math.h"
 
@@ -52,6 +50,7 @@ __device__ __forceinline__ void specvol_derivs(double T, double S, double p, dou
 __device__ __forceinline__ double cube(double x) { return (x * x) * x; }
 
 // epbl_find_mstar (rdb_ocean_epbl.F90:630-688).
+template <bool GEN>
 __device__ __forceinline__ double find_mstar(const EpblParams& c, double b0, double ustar, double bld, double absf) {
   double mstar;
   const double absf_floor = fmx(absf, 1.0e-20);
@@ -61,7 +60,7 @@ __device__ __forceinline__ double find_mstar(const EpblParams& c, double b0, dou
     if (ustar > absf_floor * bld) mstar_n = c.c_ek * sm::log(ustar / (absf_floor * fmx(bld, 1.0e-10)));
     mstar = fmx(mstar_s, fmn(1.25, mstar_n));
     if (c.mstar_cap > 0.0) mstar = fmn(c.mstar_cap, mstar);
-  } else if (c.mstar_scheme == RDB_EPBL_MSTAR_RH18) {
+  } else if (GEN && c.mstar_scheme == RDB_EPBL_MSTAR_RH18) {
     const double msn_term = c.cn2 * sm::exp(c.cn3 * bld * absf / ustar);
     const double mstar_n = c.cn1 * msn_term / (1.0 + msn_term);
     const double bp = fmx(0.0, b0);
@@ -84,10 +83,11 @@ __device__ __forceinline__ double find_mstar(const EpblParams& c, double b0, dou
 }
 
 // epbl_mixlen_shape (:690-714).
+template <bool GEN>
 __device__ __forceinline__ double mixlen_shape(const EpblParams& c, double z, double mld_guess) {
   if (!c.mld_iteration || c.translay >= 1.0 || c.translay < 0.0 || mld_guess <= 0.0) return 1.0;
   const double fr = fmx(0.0, (mld_guess - z) / mld_guess);
-  if (c.mixlen_exponent == 2.0) return c.translay + (1.0 - c.translay) * fr * fr;
+  if (!GEN || c.mixlen_exponent == 2.0) return c.translay + (1.0 - c.translay) * fr * fr;
   return c.translay + (1.0 - c.translay) * sm::pow(fr, c.mixlen_exponent);
 }
 
@@ -159,9 +159,10 @@ __device__ __noinline__ double lt_enhance(const EpblParams& c, double la, double
   return mstar * enh;
 }
 
+template <bool GEN>
 __device__ __forceinline__ double vstar_of(const EpblParams& c, double tke_here, double conv_perel, double htot,
                                            double mld_guess, double ustar, double dt, double rho0) {
-  if (c.vstar_scheme == RDB_EPBL_VSTAR_RH18) {
+  if (GEN && c.vstar_scheme == RDB_EPBL_VSTAR_RH18) {
     const double surf_scale = fmx(0.05, 1.0 - htot / mld_guess);
     return c.vstar_scale_fac * surf_scale *
            (c.vstar_surf_fac * ustar + cbrt_kahan(c.wstar_ustar_coef * conv_perel / (dt * rho0)));
@@ -204,258 +205,558 @@ __device__ __forceinline__ LevelPrep level_prep(double hk, double T, double S, d
   return q;
 }
 
+// The state of one downward sweep between two interfaces; A is the layer
+// above the next interface.
+struct EpblSweep {
+  double mech_tke, conv_perel;
+  double hA, pres, hp_a, dpe_t_a, dpe_s_a, dch_t_a, dch_s_a, th_a, sh_a, te_lag, se_lag, kddt_prev;
+  double htot, z_int, pres_int, mld_output;
+  double A_t0, A_s0, A_dch_t, A_dch_s;
+  double d_wind, d_conv, d_forcing, d_mixing, d_mdecay, d_cdecay;
+  bool sfc_connected;
+};
+
+// Values of one column that every sweep uses.
+struct EpblColumn {
+  double h_sum, absf, idecay, ustar, rho0, dt, mld_guess;
+};
+
+// h, T and S of one level, loaded ahead of the sweep.
+struct EpblLevel {
+  double h, T, S;
+};
+
+// The levels of one lane's column that its sweep comes to next, a block of N
+// in LDS.  (Loaded a level or two ahead into registers they cost a full
+// memory round trip an interface: the compiler waits for every load in
+// flight where the slots rotate, and for the stores of kd_int with them.)
+template <int N>
+struct EpblLevels {
+  const StateView& s;
+  double* slot;  // this lane's first of 3 N, 64 apart
+  int p, base;   // levels base .. base + N - 1 are held
+  __device__ __forceinline__ EpblLevels(const StateView& sv, double* lds, int col)
+      : s(sv), slot(lds + (threadIdx.x & 63)), p(col), base(-N) {}
+  __device__ __forceinline__ EpblLevel at(int k) {
+    const int P = s.P;
+    if (k < base || k >= base + N) {
+      base = max(k - (N - 1), 0);
+      double v[3 * N];
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const int kk = min(base + j, s.nz - 1);
+        v[3 * j] = LV(s.h, kk);
+        v[3 * j + 1] = LV(s.T, kk);
+        v[3 * j + 2] = LV(s.S, kk);
+      }
+#pragma unroll
+      for (int j = 0; j < 3 * N; ++j) slot[64 * j] = v[j];
+    }
+    const double* q = slot + 192 * (k - base);
+    return EpblLevel{q[0], q[64], q[128]};
+  }
+};
+
+// One interface ki of the sweep (between the layer above, in st, and layer
+// B = ki - 1): the energy solve and the embedded forward elimination.
+// Returns whether the sweep disconnects from the surface here.
+//
+// The reference evaluates v* and K for the mechanical energy first, then, in
+// a convecting interface (pe_max < 0), again with the energy that convection
+// releases, and keeps the first only if the second would cost energy.  The
+// sign test needs neither, so it comes first and a single evaluation serves
+// both branches; the first value is formed only in that rare case.  The
+// energy of the accepted K is the same expression in both branches.
+template <bool GEN>
+__device__ __forceinline__ bool epbl_interface(const EpblParams& c, const EpblColumn& q, bool first, EpblLevel lev,
+                                               EpblSweep& st, double& kd_out) {
+  const double G = GRAVITY, nstar = c.nstar, rho0 = q.rho0, dt = q.dt;
+  const double hB = lev.h;
+  const LevelPrep B = level_prep(hB, lev.T, lev.S, rho0, st.pres);
+  const double h_ka = st.hA + H_NEGLECT;
+  const double h_kb = hB + H_NEGLECT;
+  bool sfc_disconnect = false;
+  // with no mechanical TKE left the decay changes nothing:
+  // (1 - e) * 0 and 0 * e are 0 for the finite e in (0, 1]
+  if (st.mech_tke != 0.0) {
+    const double exp_kh = sm::exp(-h_ka * q.idecay);
+    st.d_mdecay = st.d_mdecay + (1.0 - exp_kh) * st.mech_tke;
+    st.mech_tke = st.mech_tke * exp_kh;
+  }
+  double nstar_fc = nstar;
+  if (st.conv_perel > 0.0 && q.absf > 0.0) {
+    const double ah = q.absf * st.htot;
+    nstar_fc = nstar * st.conv_perel / (st.conv_perel + 0.2 * sqrt(0.5 * dt * rho0 * cube(ah) * st.conv_perel));
+  }
+  const double tot_tke = st.mech_tke + nstar_fc * st.conv_perel;
+  const double dt_h = dt / fmx(0.5 * (h_ka + h_kb), 1.0e-15 * q.h_sum);
+  double kd_val;
+  if (tot_tke <= 0.0 &&
+      0.0 <= (B.dch_t + st.A_dch_t) * (st.A_t0 - B.t0) + (B.dch_s + st.A_dch_s) * (st.A_s0 - B.s0)) {
+    kd_val = 0.0;
+    sfc_disconnect = true;
+  } else {
+    const double hp_b = h_kb;
+    const double th_b = h_kb * B.t0, sh_b = h_kb * B.s0;
+    const double hps = st.hp_a + hp_b;
+    const double bdt1 = st.hp_a * hp_b;
+    const double dt_c = st.hp_a * th_b - hp_b * st.th_a;
+    const double ds_c = st.hp_a * sh_b - hp_b * st.sh_a;
+    double pec_core = hp_b * (st.dpe_t_a * dt_c + st.dpe_s_a * ds_c) - st.hp_a * (B.dpe_t * dt_c + B.dpe_s * ds_c);
+    const double colht_core =
+        hp_b * (st.dch_t_a * dt_c + st.dch_s_a * ds_c) - st.hp_a * (B.dch_t * dt_c + B.dch_s * ds_c);
+    if (colht_core < 0.0) pec_core = pec_core - st.pres_int * colht_core;
+    const double pe_max = pec_core / (bdt1 * hps);
+    const bool conv = pe_max < 0.0;
+    const double hb_hs = (q.h_sum - st.z_int) / q.h_sum;
+    const double hbs = fmn(hb_hs, mixlen_shape<GEN>(c, st.z_int, q.mld_guess));
+    auto kd_for = [&](double tke) -> double {
+      if (!(tke > 0.0)) return 0.0;
+      const double vstar = vstar_of<GEN>(c, tke, st.conv_perel, st.htot, q.mld_guess, q.ustar, dt, rho0);
+      return kd_of(c, vstar, st.htot, hbs, q.absf);
+    };
+    kd_val = kd_for(st.mech_tke + c.wstar_ustar_coef * (conv ? st.conv_perel - pe_max : st.conv_perel));
+    const double dkddt = kd_val * dt_h;
+    const double num = pec_core * dkddt, den = bdt1 * (bdt1 + dkddt * hps);
+    double energy = num / den;
+    if (conv) {
+      if (energy > 0.0) {
+        kd_val = kd_for(st.mech_tke + c.wstar_ustar_coef * st.conv_perel);
+        const double dk0 = kd_val * dt_h;
+        energy = pec_core * dk0 / (bdt1 * (bdt1 + dk0 * hps));
+      }
+      st.conv_perel = st.conv_perel - energy;
+      st.d_conv = st.d_conv - nstar * energy;
+      if (st.sfc_connected) st.mld_output = st.mld_output + hB;
+    } else {
+      double frac_bl = 1.0;
+      if (!((num <= tot_tke * den) || (pec_core <= 0.0))) {
+        kd_val = ((bdt1 * bdt1) * tot_tke) / (dt_h * (pec_core - bdt1 * hps * tot_tke));
+        energy = tot_tke;
+        frac_bl = tot_tke * den / num;
+      }
+      if (st.sfc_connected) st.mld_output = st.mld_output + frac_bl * hB;
+      if (frac_bl < 1.0) sfc_disconnect = true;
+      double r_reduc = 0.0;
+      if (tot_tke > 0.0 && tot_tke > energy) r_reduc = (tot_tke - energy) / tot_tke;
+      st.d_mixing = st.d_mixing + energy;
+      st.d_cdecay = st.d_cdecay + (1.0 - r_reduc) * (nstar - nstar_fc) * st.conv_perel;
+      st.mech_tke = r_reduc * st.mech_tke;
+      st.conv_perel = r_reduc * st.conv_perel;
+    }
+  }
+  kd_out = kd_val;
+  const double kddt_cur = kd_val * dt_h;
+  const double b1 = 1.0 / (st.hp_a + kddt_cur);
+  const double c1 = kddt_cur * b1;
+  if (first) {
+    st.te_lag = b1 * (h_ka * st.A_t0);
+    st.se_lag = b1 * (h_ka * st.A_s0);
+  } else {
+    st.te_lag = b1 * (h_ka * st.A_t0 + st.kddt_prev * st.te_lag);
+    st.se_lag = b1 * (h_ka * st.A_s0 + st.kddt_prev * st.se_lag);
+  }
+  st.hp_a = h_kb + (st.hp_a * b1) * kddt_cur;
+  st.dpe_t_a = B.dpe_t + c1 * st.dpe_t_a;
+  st.dpe_s_a = B.dpe_s + c1 * st.dpe_s_a;
+  st.dch_t_a = B.dch_t + c1 * st.dch_t_a;
+  st.dch_s_a = B.dch_s + c1 * st.dch_s_a;
+  st.th_a = h_kb * B.t0 + kddt_cur * st.te_lag;
+  st.sh_a = h_kb * B.s0 + kddt_cur * st.se_lag;
+  st.kddt_prev = kddt_cur;
+  if (sfc_disconnect) {
+    st.htot = hB;
+    st.sfc_connected = false;
+  } else {
+    st.htot = st.htot + hB;
+  }
+  st.z_int = st.z_int + hB;
+  st.pres_int = st.pres_int + G * rho0 * hB;
+  st.hA = hB;
+  st.A_t0 = B.t0;
+  st.A_s0 = B.s0;
+  st.A_dch_t = B.dch_t;
+  st.A_dch_s = B.dch_s;
+  return sfc_disconnect;
+}
+
+// What the sweeps of one column start from, and the surface forcing.
+struct EpblStart {
+  int k_sfc;
+  double h_sfc, pres0, b0, ctke_sfc, mech_in, lt_ustokes, lt_kphil;
+  LevelPrep top;
+};
+
+// The surface layer, column depth and forcing of packed column p
+// (:1087-1226).
+template <bool GEN>
+__device__ __forceinline__ EpblStart epbl_start(const StateView& s, const EpblParams& c, const double* fcor,
+                                                double rho0, double cp, double dt, int p, EpblColumn& q) {
+  const int P = s.P, nz = s.nz;
+  const double G = GRAVITY;
+  EpblStart a;
+  // the surface layer: the first live layer counting down from the top
+  a.k_sfc = nz - 1;
+  for (int k = nz - 1; k >= 0; --k)
+    if (LV(s.h, k) > H_VANISHED) {
+      a.k_sfc = k;
+      break;
+    }
+  // (eight loads a round: the sum is serial, the loads are not)
+  double h_sum = 0.0;
+  for (int k0 = a.k_sfc; k0 >= 0; k0 -= 8) {
+    double hh[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) hh[j] = LV(s.h, max(k0 - j, 0));
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (k0 - j >= 0) h_sum = h_sum + hh[j];
+  }
+  q.h_sum = h_sum + H_NEGLECT;
+  a.h_sfc = LV(s.h, a.k_sfc);
+  a.pres0 = 0.0;
+  a.top = level_prep(a.h_sfc, LV(s.T, a.k_sfc), LV(s.S, a.k_sfc), rho0, a.pres0);
+  const double dmass_s = rho0 * a.h_sfc;
+  const double pmid_s = 0.0 + 0.5 * (G * dmass_s);
+  double dsv_dt_sfc, dsv_ds_sfc;
+  specvol_derivs(a.top.t0, a.top.s0, pmid_s, dsv_dt_sfc, dsv_ds_sfc);
+  const double q_t_kin = (1.0 / (rho0 * cp)) * s.Qh[p];
+  const double q_s_kin = (1.0 / rho0) * s.Qs[p];
+  a.b0 = G * rho0 * (dsv_dt_sfc * q_t_kin + dsv_ds_sfc * q_s_kin);
+  a.ctke_sfc = -(0.5 * G * (rho0 * rho0) * a.h_sfc * (q_t_kin * dt * dsv_dt_sfc + q_s_kin * dt * dsv_ds_sfc));
+  q.ustar = fmx(sqrt(s.tau_tot[p] / rho0), c.ustar_min);
+  const double f = fcor[p];
+  q.absf = sqrt((1.0 - c.omega_frac) * (f * f) + c.omega_frac * 4.0 * (c.omega * c.omega));
+  q.idecay = c.tke_decay * q.absf / q.ustar;
+  q.rho0 = rho0;
+  q.dt = dt;
+  a.mech_in = dt * rho0 * cube(q.ustar);
+  a.lt_ustokes = a.lt_kphil = 0.0;
+  if (GEN && c.use_lt) lf17_wave_state(q.ustar, rho0, a.lt_ustokes, a.lt_kphil);
+  return a;
+}
+
+// The top of a sweep for the guess q.mld_guess (:1290-1350).
+template <bool GEN>
+__device__ __forceinline__ void epbl_begin(const EpblParams& c, const EpblColumn& q, const EpblStart& a,
+                                           EpblSweep& st, double& la_val) {
+  double mstar_val = find_mstar<GEN>(c, a.b0, q.ustar, q.mld_guess, q.absf);
+  if (GEN && c.use_lt) {
+    la_val = lf17_la(q.ustar, c.la_frac_hbl * q.mld_guess, a.lt_ustokes, a.lt_kphil);
+    mstar_val = lt_enhance(c, la_val, a.b0, q.ustar, q.mld_guess, q.absf, mstar_val);
+  }
+  st.mech_tke = mstar_val * a.mech_in;
+  st.d_wind = st.mech_tke;
+  st.d_conv = st.d_forcing = st.d_mixing = st.d_mdecay = st.d_cdecay = 0.0;
+  if (a.ctke_sfc <= 0.0) {
+    const double forcing_clip = fmx(a.ctke_sfc, -st.mech_tke);
+    st.mech_tke = st.mech_tke + forcing_clip;
+    st.conv_perel = 0.0;
+    st.d_forcing = forcing_clip;
+  } else {
+    st.conv_perel = a.ctke_sfc;
+    st.d_conv = c.nstar * a.ctke_sfc;
+  }
+  st.hA = a.h_sfc;
+  st.A_t0 = a.top.t0;
+  st.A_s0 = a.top.s0;
+  st.A_dch_t = a.top.dch_t;
+  st.A_dch_s = a.top.dch_s;
+  st.pres = a.pres0;
+  st.hp_a = a.h_sfc + H_NEGLECT;
+  st.dpe_t_a = a.top.dpe_t;
+  st.dpe_s_a = a.top.dpe_s;
+  st.dch_t_a = a.top.dch_t;
+  st.dch_s_a = a.top.dch_s;
+  st.th_a = st.hp_a * a.top.t0;
+  st.sh_a = st.hp_a * a.top.s0;
+  st.te_lag = st.se_lag = st.kddt_prev = 0.0;
+  st.htot = a.h_sfc;
+  st.z_int = a.h_sfc;
+  st.pres_int = GRAVITY * q.rho0 * a.h_sfc;
+  st.mld_output = a.h_sfc;
+  st.sfc_connected = true;
+}
+
+// The MLD root-finder (:1625-1641) between two guesses.
+struct EpblRoot {
+  double min_mld, max_mld, dmld_min, dmld_max;
+  bool have_min, have_max;
+  // the guess after iteration it, whose sweep for `guess` found `found`
+  __device__ __forceinline__ double next(const EpblParams& c, int it, double guess, double found) {
+    if (found > guess) {
+      min_mld = guess;
+      dmld_min = found - guess;
+      have_min = true;
+    } else {
+      max_mld = guess;
+      dmld_max = found - guess;
+      have_max = true;
+    }
+    if (c.mld_bisection) return 0.5 * (min_mld + max_mld);
+    if (have_min && have_max && it > 2 && ((it - 1) % 4) > 0)
+      return min_mld + dmld_min * (max_mld - min_mld) / (dmld_min - dmld_max);
+    if (found > min_mld && found < max_mld) return found;
+    return 0.5 * (min_mld + max_mld);
+  }
+};
+
+// Whether iteration it, with this guess and this result, is the last.
+__device__ __forceinline__ bool epbl_last(const EpblParams& c, int it, double guess, double found) {
+  return !c.mld_iteration || it == c.mld_max_its || fabs(found - guess) < c.mld_tol;
+}
+
+__device__ __forceinline__ void epbl_store(const StateView& s, const EpblParams& c, const EpblView& e, int p,
+                                           const EpblSweep& st, double mld, double la, double dt) {
+  const int P = s.P;
+  e.mld[p] = mld;
+  e.la[p] = la;
+  if (c.tke_diags) {
+    LV(e.tke, 0) = st.d_wind / dt;
+    LV(e.tke, 1) = st.d_conv / dt;
+    LV(e.tke, 2) = st.d_forcing / dt;
+    LV(e.tke, 3) = st.d_mixing / dt;
+    LV(e.tke, 4) = st.d_mdecay / dt;
+    LV(e.tke, 5) = st.d_cdecay / dt;
+  }
+}
+
+// A sweep that is still connected where less than the root finder's
+// tolerance is left below, in at least this many layers, leaves its column to
+// k_epbl_bed.
+constexpr int BED_LEVELS = 12;
+// Guesses that k_epbl_bed tries at a time, a wavefront each.
+constexpr int BED_WAVES = 8;
+
 }  // namespace
 
 // The EPBL solve for the packed columns [p0, p1): kd_int, MLD, B0, La and
-// the TKE ledger of each (free surface, no penetrating shortwave).
+// the TKE ledger of each (free surface, no penetrating shortwave).  One lane
+// per column: a serial chain of about 550 vector instructions an interface,
+// 2 us of it at one or two wavefronts a SIMD, so the longest chain bounds the
+// kernel.  On 480 x 360 x 75 (121 000 wet columns) one solve took 1.66 ms,
+// eight sweeps of 74 interfaces in the columns over fillers; now 0.22 ms here
+// and 0.49 ms in k_epbl_bed.  What gave it: those columns' sweeps side by
+// side; the last guess's sweep carried on where it stopped instead of
+// repeated; one evaluation of v* and K an interface; levels through LDS.
+// (Branch-free exp and cbrt, to leave the compiler longer blocks, cost
+// 0.04 ms; two waves a SIMD need the 256-register cap.)
+template <bool GEN>
 __global__ void __launch_bounds__(64, 2) k_epbl(StateView s, EpblParams c, EpblView e, const double* __restrict__ fcor,
-                                               double rho0, double cp, double dt, int p0, int p1) {
+                                             double rho0, double cp, double dt, int p0, int p1) {
+  __shared__ double lds[3 * 8 * 64];
   const int p = p0 + blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= p1) return;
   const int P = s.P, nz = s.nz;
-  const double G = GRAVITY, nstar = c.nstar;
-  // the surface layer: the first live layer counting down from the top
-  int k_sfc = nz - 1;
-  for (int k = nz - 1; k >= 0; --k)
-    if (LV(s.h, k) > H_VANISHED) {
-      k_sfc = k;
-      break;
-    }
-  double h_sum = 0.0;
-  for (int k = k_sfc; k >= 0; --k) h_sum = h_sum + LV(s.h, k);
-  h_sum = h_sum + H_NEGLECT;
-  const double h_sfc = LV(s.h, k_sfc);
-  double pres0 = 0.0;
-  const LevelPrep top = level_prep(h_sfc, LV(s.T, k_sfc), LV(s.S, k_sfc), rho0, pres0);
-  const double dmass_s = rho0 * h_sfc;
-  const double pmid_s = 0.0 + 0.5 * (G * dmass_s);
-  double dsv_dt_sfc, dsv_ds_sfc;
-  specvol_derivs(top.t0, top.s0, pmid_s, dsv_dt_sfc, dsv_ds_sfc);
-  // forcing (:1185-1226)
-  const double q_t_kin = (1.0 / (rho0 * cp)) * s.Qh[p];
-  const double q_s_kin = (1.0 / rho0) * s.Qs[p];
-  const double b0 = G * rho0 * (dsv_dt_sfc * q_t_kin + dsv_ds_sfc * q_s_kin);
-  e.b0[p] = b0;
-  const double ctke_sfc = -(0.5 * G * (rho0 * rho0) * h_sfc * (q_t_kin * dt * dsv_dt_sfc + q_s_kin * dt * dsv_ds_sfc));
-  const double ustar = fmx(sqrt(s.tau_tot[p] / rho0), c.ustar_min);
-  const double f = fcor[p];
-  const double absf = sqrt((1.0 - c.omega_frac) * (f * f) + c.omega_frac * 4.0 * (c.omega * c.omega));
-  const double idecay = c.tke_decay * absf / ustar;
-  const double mech_in = dt * rho0 * cube(ustar);
-  double la_val = 0.0, lt_ustokes = 0.0, lt_kphil = 0.0;
-  if (c.use_lt) lf17_wave_state(ustar, rho0, lt_ustokes, lt_kphil);
-  double d_wind = 0.0, d_conv = 0.0, d_forcing = 0.0, d_mixing = 0.0, d_mdecay = 0.0, d_cdecay = 0.0;
+  EpblLevels<8> levels(s, lds, p);
+  EpblColumn q;
+  const EpblStart a = epbl_start<GEN>(s, c, fcor, rho0, cp, dt, p, q);
+  e.b0[p] = a.b0;
+  double la_val = 0.0;
+  EpblSweep st;
+  st.d_wind = st.d_conv = st.d_forcing = st.d_mixing = st.d_mdecay = st.d_cdecay = 0.0;
   double mld_found = 0.0;
 
-  if (s.wet[p] <= 0.0 || h_sum <= 2.0 * H_NEGLECT) {
+  if (s.wet[p] <= 0.0 || q.h_sum <= 2.0 * H_NEGLECT) {
     for (int k = 0; k <= nz; ++k) LV(e.kd, k) = 0.0;
   } else {
-    double min_mld = 0.0, max_mld = h_sum, dmld_min = 0.0, dmld_max = 0.0;
-    bool have_min = false, have_max = false;
-    double mld_guess = 0.5 * (min_mld + max_mld);
-    if (c.mld_use_prev_guess && e.mld[p] > 0.0) mld_guess = fmn(e.mld[p], max_mld);
-    const int n_its = c.mld_iteration ? c.mld_max_its : 1;
-    for (int k = k_sfc + 1; k <= nz; ++k) LV(e.kd, k) = 0.0;
+    EpblRoot root{0.0, q.h_sum, 0.0, 0.0, false, false};
+    q.mld_guess = 0.5 * (root.min_mld + root.max_mld);
+    if (c.mld_use_prev_guess && e.mld[p] > 0.0) q.mld_guess = fmn(e.mld[p], root.max_mld);
+    for (int k = a.k_sfc + 1; k <= nz; ++k) LV(e.kd, k) = 0.0;
     LV(e.kd, 0) = 0.0;
-    // One sweep of the column for the guess mld_guess.  A guess that is not
-    // the last one only needs the MLD, which stops growing once the sweep
-    // disconnects from the surface: those sweeps (FULL = false) stop there
-    // and write nothing.  The last guess is swept in full (kd_int and the
-    // TKE ledger); both kinds run the same arithmetic down to the
-    // disconnect, so the MLD they find is the same to the bit.
-    auto sweep = [&](auto full_tag, double mld_guess) -> double {
-      constexpr bool FULL = decltype(full_tag)::value;
-      d_wind = d_conv = d_forcing = d_mixing = d_mdecay = d_cdecay = 0.0;
-      double mstar_val = find_mstar(c, b0, ustar, mld_guess, absf);
-      if (c.use_lt) {
-        la_val = lf17_la(ustar, c.la_frac_hbl * mld_guess, lt_ustokes, lt_kphil);
-        mstar_val = lt_enhance(c, la_val, b0, ustar, mld_guess, absf, mstar_val);
-      }
-      double mech_tke = mstar_val * mech_in;
-      d_wind = mech_tke;
-      double conv_perel;
-      if (ctke_sfc <= 0.0) {
-        const double forcing_clip = fmx(ctke_sfc, -mech_tke);
-        mech_tke = mech_tke + forcing_clip;
-        conv_perel = 0.0;
-        d_forcing = forcing_clip;
-      } else {
-        conv_perel = ctke_sfc;
-        d_conv = nstar * ctke_sfc;
-      }
-      // sweep initialisation (:1330-1350); A is the layer above the
-      // interface, B the one below
-      double hA = h_sfc;
-      LevelPrep A = top;
-      double pres = pres0;
-      double h_ka = hA + H_NEGLECT;
-      double hp_a = h_ka;
-      double dpe_t_a = A.dpe_t, dpe_s_a = A.dpe_s, dch_t_a = A.dch_t, dch_s_a = A.dch_s;
-      double th_a = h_ka * A.t0, sh_a = h_ka * A.s0;
-      double te_lag = 0.0, se_lag = 0.0, kddt_prev = 0.0;
-      double htot = hA, z_int = hA, pres_int = G * rho0 * hA;
-      double mld_output = hA;
-      bool sfc_connected = true;
-      for (int ki = k_sfc; ki >= 1; --ki) {
-        const int kb = ki - 1;
-        const double hB = LV(s.h, kb);
-        const LevelPrep B = level_prep(hB, LV(s.T, kb), LV(s.S, kb), rho0, pres);
-        h_ka = hA + H_NEGLECT;
-        const double h_kb = hB + H_NEGLECT;
-        bool sfc_disconnect = false;
-        // with no mechanical TKE left the decay changes nothing:
-        // (1 - e) * 0 and 0 * e are 0 for the finite e in (0, 1]
-        if (mech_tke != 0.0) {
-          const double exp_kh = sm::exp(-h_ka * idecay);
-          d_mdecay = d_mdecay + (1.0 - exp_kh) * mech_tke;
-          mech_tke = mech_tke * exp_kh;
+    // A guess only needs the MLD, which stops growing once its sweep
+    // disconnects from the surface: each sweep stops there.  kd_int is
+    // written as the sweep goes (a later guess overwrites it), so the sweep
+    // of the last guess only has to be carried on from where it stopped,
+    // below.
+    int ki = a.k_sfc;
+    for (int it = 1;; ++it) {
+      epbl_begin<GEN>(c, q, a, st, la_val);
+      for (ki = a.k_sfc; ki >= 1; --ki) {
+        if (it == 1 && c.mld_iteration && ki > BED_LEVELS && q.h_sum - st.z_int < c.mld_tol) {
+          // connected to the bottom of the water, fillers below
+          e.bed_list[atomicAdd(e.bed_count, 1u)] = p;
+          return;
         }
-        double nstar_fc = nstar;
-        if (conv_perel > 0.0 && absf > 0.0) {
-          const double ah = absf * htot;
-          nstar_fc = nstar * conv_perel / (conv_perel + 0.2 * sqrt(0.5 * dt * rho0 * cube(ah) * conv_perel));
+        double kd;
+        const bool dis = epbl_interface<GEN>(c, q, ki == a.k_sfc, levels.at(ki - 1), st, kd);
+        LV(e.kd, ki) = kd;
+        if (dis) {
+          --ki;
+          break;
         }
-        const double tot_tke = mech_tke + nstar_fc * conv_perel;
-        const double dt_h = dt / fmx(0.5 * (h_ka + h_kb), 1.0e-15 * h_sum);
-        double kd_val;
-        if (tot_tke <= 0.0 && 0.0 <= (B.dch_t + A.dch_t) * (A.t0 - B.t0) + (B.dch_s + A.dch_s) * (A.s0 - B.s0)) {
-          kd_val = 0.0;
-          sfc_disconnect = true;
-        } else {
-          double tke_here = mech_tke + c.wstar_ustar_coef * conv_perel;
-          const double hb_hs = (h_sum - z_int) / h_sum;
-          const double hbs = fmn(hb_hs, mixlen_shape(c, z_int, mld_guess));
-          double kd_g0 = 0.0;
-          if (tke_here > 0.0) {
-            const double vstar = vstar_of(c, tke_here, conv_perel, htot, mld_guess, ustar, dt, rho0);
-            kd_g0 = kd_of(c, vstar, htot, hbs, absf);
+      }
+      mld_found = st.mld_output;
+      if (epbl_last(c, it, q.mld_guess, mld_found)) break;
+      q.mld_guess = root.next(c, it, q.mld_guess, mld_found);
+    }
+    // The last guess's sweep goes on to the bed.  Every lane walks from the
+    // wavefront's highest open interface, so that a level stays one
+    // coalesced access, and joins at its own.
+    int top_open = nz - 1;
+    while (top_open >= 1 && !__any(ki >= top_open)) --top_open;
+    for (int k = top_open; k >= 1; --k) {
+      if (k <= ki) {
+        double kd;
+        epbl_interface<GEN>(c, q, k == a.k_sfc, levels.at(k - 1), st, kd);
+        LV(e.kd, k) = kd;
+      }
+    }
+    st.d_mdecay = st.d_mdecay + st.mech_tke;
+    st.d_cdecay = st.d_cdecay + c.nstar * st.conv_perel;
+  }
+  epbl_store(s, c, e, p, st, mld_found, la_val, dt);
+}
+
+// The columns that are mixed to the bottom of the water and hold a stack of
+// fillers below it (two or three live layers of 75, above all): the root
+// finder halves its way to the column depth, about eight sweeps of the whole
+// column one after the other, eight times the length of any other column's
+// chain (592 interfaces of 75 layers).  Each of those sweeps finds the whole
+// column, so the guesses are known beforehand: a workgroup takes 64 columns
+// and each wavefront sweeps one guess of the sequence that results when
+// every sweep finds the column's thickness.  Then the first wavefront
+// replays the root finder on the results; a guess that is not the foreseen
+// one (a sweep found something else) is swept there.  The guesses, their
+// sweeps and the order of the decisions are the sequential ones, so the bits
+// are.
+template <bool GEN>
+__global__ void __launch_bounds__(64 * BED_WAVES) k_epbl_bed(StateView s, EpblParams c, EpblView e,
+                                                             const double* __restrict__ fcor, double rho0, double cp,
+                                                             double dt) {
+  __shared__ double lds[BED_WAVES][3 * 4 * 64], sh_guess[BED_WAVES][64], sh_found[BED_WAVES][64];
+  __shared__ int sh_owner[64];
+  const int P = s.P, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = (int)*e.bed_count;
+  for (int i0 = blockIdx.x * 64; i0 < n; i0 += gridDim.x * 64) {
+    const bool on = i0 + lane < n;
+    const int p = e.bed_list[on ? i0 + lane : i0];
+    EpblColumn q;
+    const EpblStart a = epbl_start<GEN>(s, c, fcor, rho0, cp, dt, p, q);
+    EpblLevels<4> levels(s, lds[wave], p);
+    EpblRoot root{0.0, q.h_sum, 0.0, 0.0, false, false};
+    double guess = 0.5 * (root.min_mld + root.max_mld);
+    if (c.mld_use_prev_guess && e.mld[p] > 0.0) guess = fmn(e.mld[p], root.max_mld);
+    int it = 1;
+    // this wavefront's guess of the foreseen sequence: iteration 1 + wave,
+    // where every sweep adds up the column (h_sum: the same sum in the same
+    // order, H_NEGLECT vanishes in it)
+    bool foreseen = on;
+    double my_guess = guess;
+    {
+      EpblRoot r = root;
+      for (int j = 0; j < wave && foreseen; ++j) {
+        if (epbl_last(c, 1 + j, my_guess, q.h_sum))
+          foreseen = false;
+        else
+          my_guess = r.next(c, 1 + j, my_guess, q.h_sum);
+      }
+    }
+    // kd_int of this sweep, until it is known whose guess is the last: a
+    // column of the scratch arrays fa and fb, if there are that many
+    const long long slot = (long long)i0 * BED_WAVES + 64 * wave + lane;
+    foreseen = foreseen && slot < 2LL * P;
+    double* const kds = slot < P ? s.fa + slot : s.fb + (slot < 2LL * P ? slot - P : 0);
+    // One sweep loop serves every phase (three copies of it spill): first
+    // each wavefront's foreseen guess, then the first wavefront's guesses
+    // that were not foreseen, then the last guess's sweep on to the bed.
+    EpblSweep st;
+    double la_val = 0.0;
+    int ki = 0, k_kept = 0;
+    int phase = 0;
+    bool go = foreseen, decided = !on;
+    double* kd_to = kds;
+    q.mld_guess = my_guess;
+    for (;;) {
+      if (go) {
+        if (phase < 2) {
+          epbl_begin<GEN>(c, q, a, st, la_val);
+          ki = a.k_sfc;
+        }
+        for (; ki >= 1; --ki) {
+          double kd;
+          const bool dis = epbl_interface<GEN>(c, q, ki == a.k_sfc, levels.at(ki - 1), st, kd);
+          kd_to[(size_t)ki * (size_t)P] = kd;
+          if (dis && phase < 2) {
+            --ki;
+            break;
           }
-          const double hp_b = h_kb;
-          const double th_b = h_kb * B.t0, sh_b = h_kb * B.s0;
-          const double hps = hp_a + hp_b;
-          const double bdt1 = hp_a * hp_b;
-          const double dt_c = hp_a * th_b - hp_b * th_a;
-          const double ds_c = hp_a * sh_b - hp_b * sh_a;
-          double pec_core = hp_b * (dpe_t_a * dt_c + dpe_s_a * ds_c) - hp_a * (B.dpe_t * dt_c + B.dpe_s * ds_c);
-          const double colht_core = hp_b * (dch_t_a * dt_c + dch_s_a * ds_c) - hp_a * (B.dch_t * dt_c + B.dch_s * ds_c);
-          if (colht_core < 0.0) pec_core = pec_core - pres_int * colht_core;
-          const double dkddt = kd_g0 * dt_h;
-          const double pe_max = pec_core / (bdt1 * hps);
-          if (pe_max < 0.0) {
-            tke_here = mech_tke + c.wstar_ustar_coef * (conv_perel - pe_max);
-            kd_val = 0.0;
-            if (tke_here > 0.0) {
-              const double vstar = vstar_of(c, tke_here, conv_perel, htot, mld_guess, ustar, dt, rho0);
-              kd_val = kd_of(c, vstar, htot, hbs, absf);
+        }
+      }
+      if (phase == 2) break;
+      if (phase == 0) {
+        sh_guess[wave][lane] = my_guess;
+        sh_found[wave][lane] = foreseen ? st.mld_output : -1.0;
+        k_kept = ki;  // interfaces k_sfc .. k_kept + 1 are in kds
+        kd_to = e.kd + p;
+        phase = 1;
+        go = false;
+        __syncthreads();
+      }
+      if (wave == 0) {
+        // replay the root finder on the results at hand
+        while (!decided) {
+          const int w = it - 1;
+          double f = st.mld_output;
+          const bool swept = go;
+          if (!swept) {
+            if (!(w < BED_WAVES && sh_found[w][lane] >= 0.0 && sh_guess[w][lane] == guess)) {
+              q.mld_guess = guess;
+              go = true;
+              break;
             }
-            const double pe_g0 = pec_core * dkddt / (bdt1 * (bdt1 + dkddt * hps));
-            double dpe_conv = pec_core * (kd_val * dt_h) / (bdt1 * (bdt1 + (kd_val * dt_h) * hps));
-            if (dpe_conv > 0.0) {
-              kd_val = kd_g0;
-              dpe_conv = pe_g0;
-            }
-            conv_perel = conv_perel - dpe_conv;
-            d_conv = d_conv - nstar * dpe_conv;
-            if (sfc_connected) mld_output = mld_output + hB;
+            f = sh_found[w][lane];
+          }
+          go = false;
+          if (epbl_last(c, it, guess, f)) {
+            sh_owner[lane] = swept ? BED_WAVES : w;
+            decided = true;
           } else {
-            double tke_used, frac_bl;
-            if ((pec_core * dkddt <= tot_tke * (bdt1 * (bdt1 + dkddt * hps))) || (pec_core <= 0.0)) {
-              kd_val = kd_g0;
-              tke_used = pec_core * dkddt / (bdt1 * (bdt1 + dkddt * hps));
-              frac_bl = 1.0;
-            } else {
-              kd_val = ((bdt1 * bdt1) * tot_tke) / (dt_h * (pec_core - bdt1 * hps * tot_tke));
-              tke_used = tot_tke;
-              frac_bl = tot_tke * (bdt1 * (bdt1 + dkddt * hps)) / (pec_core * dkddt);
-            }
-            if (sfc_connected) mld_output = mld_output + frac_bl * hB;
-            if (frac_bl < 1.0) sfc_disconnect = true;
-            double r_reduc = 0.0;
-            if (tot_tke > 0.0 && tot_tke > tke_used) r_reduc = (tot_tke - tke_used) / tot_tke;
-            d_mixing = d_mixing + tke_used;
-            d_cdecay = d_cdecay + (1.0 - r_reduc) * (nstar - nstar_fc) * conv_perel;
-            mech_tke = r_reduc * mech_tke;
-            conv_perel = r_reduc * conv_perel;
+            guess = root.next(c, it, guess, f);
+            ++it;
           }
         }
-        if (!FULL && sfc_disconnect) return mld_output;  // the MLD is final
-        if (FULL) LV(e.kd, ki) = kd_val;
-        const double kddt_cur = kd_val * dt_h;
-        const double b1 = 1.0 / (hp_a + kddt_cur);
-        const double c1 = kddt_cur * b1;
-        if (ki == k_sfc) {
-          te_lag = b1 * (h_ka * A.t0);
-          se_lag = b1 * (h_ka * A.s0);
-        } else {
-          const double te_new = b1 * (h_ka * A.t0 + kddt_prev * te_lag);
-          const double se_new = b1 * (h_ka * A.s0 + kddt_prev * se_lag);
-          te_lag = te_new;
-          se_lag = se_new;
+        if (__any(!decided)) continue;
+      }
+      __syncthreads();
+      const int owner = on ? sh_owner[lane] : -1;
+      go = owner == wave || (wave == 0 && owner == BED_WAVES);
+      if (owner == wave)
+        for (int k0 = a.k_sfc; k0 > k_kept; k0 -= 16) {
+          double v[16];
+#pragma unroll
+          for (int j = 0; j < 16; ++j) v[j] = kds[(size_t)max(k0 - j, 0) * (size_t)P];
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            if (k0 - j > k_kept) LV(e.kd, k0 - j) = v[j];
         }
-        hp_a = h_kb + (hp_a * b1) * kddt_cur;
-        dpe_t_a = B.dpe_t + c1 * dpe_t_a;
-        dpe_s_a = B.dpe_s + c1 * dpe_s_a;
-        dch_t_a = B.dch_t + c1 * dch_t_a;
-        dch_s_a = B.dch_s + c1 * dch_s_a;
-        th_a = h_kb * B.t0 + kddt_cur * te_lag;
-        sh_a = h_kb * B.s0 + kddt_cur * se_lag;
-        kddt_prev = kddt_cur;
-        if (sfc_disconnect) {
-          htot = hB;
-          sfc_connected = false;
-        } else {
-          htot = htot + hB;
-        }
-        z_int = z_int + hB;
-        pres_int = pres_int + G * rho0 * hB;
-        hA = hB;
-        A = B;
-      }
-      d_mdecay = d_mdecay + mech_tke;
-      d_cdecay = d_cdecay + nstar * conv_perel;
-      return mld_output;
-    };
-    for (int obl_it = 1; obl_it <= n_its; ++obl_it) {
-      // a guess known to be the last is swept in full at once
-      if (!c.mld_iteration || obl_it == n_its) {
-        mld_found = sweep(std::true_type{}, mld_guess);
-        break;
-      }
-      mld_found = sweep(std::false_type{}, mld_guess);
-      if (fabs(mld_found - mld_guess) < c.mld_tol) {
-        sweep(std::true_type{}, mld_guess);
-        break;
-      }
-      if (mld_found > mld_guess) {
-        min_mld = mld_guess;
-        dmld_min = mld_found - mld_guess;
-        have_min = true;
-      } else {
-        max_mld = mld_guess;
-        dmld_max = mld_found - mld_guess;
-        have_max = true;
-      }
-      if (c.mld_bisection)
-        mld_guess = 0.5 * (min_mld + max_mld);
-      else if (have_min && have_max && obl_it > 2 && ((obl_it - 1) % 4) > 0)
-        mld_guess = min_mld + dmld_min * (max_mld - min_mld) / (dmld_min - dmld_max);
-      else if (mld_found > min_mld && mld_found < max_mld)
-        mld_guess = mld_found;
-      else
-        mld_guess = 0.5 * (min_mld + max_mld);
+      phase = 2;
+    }
+    if (go) {
+      st.d_mdecay = st.d_mdecay + st.mech_tke;
+      st.d_cdecay = st.d_cdecay + c.nstar * st.conv_perel;
+      epbl_store(s, c, e, p, st, st.mld_output, la_val, dt);
+    }
+    __syncthreads();  // the next columns reuse the shared arrays
+  }
+  // the last workgroup to finish empties the list for the next solve
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();
+    if (atomicAdd(e.bed_done, 1u) == gridDim.x - 1) {
+      *e.bed_count = 0u;
+      *e.bed_done = 0u;
     }
   }
-  e.mld[p] = mld_found;
-  e.la[p] = la_val;
-  if (c.tke_diags) {
-    LV(e.tke, 0) = d_wind / dt;
-    LV(e.tke, 1) = d_conv / dt;
-    LV(e.tke, 2) = d_forcing / dt;
-    LV(e.tke, 3) = d_mixing / dt;
-    LV(e.tke, 4) = d_mdecay / dt;
-    LV(e.tke, 5) = d_cdecay / dt;
-  }
 }
+#define INST(GEN)                                                                                                 \
+  template __global__ void k_epbl<GEN>(StateView, EpblParams, EpblView, const double*, double, double, double, int, \
+                                       int);                                                                      \
+  template __global__ void k_epbl_bed<GEN>(StateView, EpblParams, EpblView, const double*, double, double, double);
+INST(false)
+INST(true)
+#undef INST
 
 // The coefficient build after the surface scheme, one pass per column from
 // the top: PP81 at each interface (when the surface scheme did not need it
