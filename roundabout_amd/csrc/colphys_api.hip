@@ -497,13 +497,24 @@ int refresh_static(rdb_colphys* h, double dt) {
     int st = refresh_static(m, dt);
     if (st) return st;
   }
-  if (!h->static_dirty) return RDB_COLPHYS_OK;
-  hipLaunchKernelGGL(colphys::k_prepare, grid1(h->n_all, 256), dim3(256), 0, h->stream, h->s, h->pr, 0, h->n_all);
+  if (!h->static_dirty && !h->uv_dirty) return RDB_COLPHYS_OK;
+  const int n = h->n_all, nd = h->n_all - h->n_wet;
+  if (h->static_dirty)
+    hipLaunchKernelGGL(colphys::k_first_live, grid1(n, 64), dim3(64), 0, h->stream, h->s, 0, n);
+  hipLaunchKernelGGL(colphys::k_prepare, dim3(grid1(n, 256).x, (unsigned)((h->nz + PREP_LEVELS) / PREP_LEVELS)),
+                     dim3(256), 0, h->stream, h->s, h->pr, 0, n);
   int st = launch_check("k_prepare");
   if (st) return st;
-  st = launch_step(h, dt, h->n_wet, h->n_all);
+  if (nd > 0 && h->cfg.use_kpp && h->pr.ri_crit > 0.0) {
+    hipLaunchKernelGGL(h->precision == RDB_COLPHYS_PREC_SPLIT ? colphys::k_dry_columns<float>
+                                                              : colphys::k_dry_columns<double>,
+                       grid1(nd, 64), dim3(64), 0, h->stream, h->s, h->pr, h->n_wet, h->n_all);
+    st = launch_check("k_dry_columns");
+  } else {
+    st = launch_step(h, dt, h->n_wet, h->n_all);
+  }
   if (st) return st;
-  h->static_dirty = false;
+  h->static_dirty = h->uv_dirty = false;
   return RDB_COLPHYS_OK;
 }
 
@@ -1069,36 +1080,38 @@ int rdb_colphys_set_field(rdb_colphys* h, const char* name, const double* data, 
     case F_LAYER:
     case F_IFACE: {
       double* dst = layer_ptr(h, name, tracer);
-      hipLaunchKernelGGL(colphys::k_pack_layer, dim3(grid1(ncol, B).x, e3), b, 0, h->stream, h->d_stage, dst, h->d_col,
+      hipLaunchKernelGGL(colphys::k_pack_layer, colphys::plane_grid(ncol, e3), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, dst, h->d_col,
                          ncol, P, e3, (long long)nx * ny);
       break;
     }
     case F_COL: {
       double* dst = layer_ptr(h, name, tracer);
-      hipLaunchKernelGGL(colphys::k_pack_layer, dim3(grid1(ncol, B).x, 1), b, 0, h->stream, h->d_stage, dst, h->d_col,
+      hipLaunchKernelGGL(colphys::k_pack_layer, colphys::plane_grid(ncol, 1), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, dst, h->d_col,
                          ncol, P, 1, (long long)nx * ny);
       break;
     }
     case F_FACE_X:
       std::copy(data, data + n, h->h_u.begin());
       if (int e = colphys::mom_face_set(h, true)) return e;
-      hipLaunchKernelGGL(colphys::k_pack_centre_x, dim3(grid1(ncol, B).x, nz), b, 0, h->stream, h->d_stage, h->s.ub,
+      hipLaunchKernelGGL(colphys::k_pack_centre_x, colphys::plane_grid(ncol, nz), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, h->s.ub,
                          h->d_col, ncol, P, nz, nx, ny);
       break;
     case F_FACE_Y:
       std::copy(data, data + n, h->h_v.begin());
       if (int e = colphys::mom_face_set(h, false)) return e;
-      hipLaunchKernelGGL(colphys::k_pack_centre_y, dim3(grid1(ncol, B).x, nz), b, 0, h->stream, h->d_stage, h->s.vb,
+      hipLaunchKernelGGL(colphys::k_pack_centre_y, colphys::plane_grid(ncol, nz), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, h->s.vb,
                          h->d_col, ncol, P, nz, nx, ny);
       break;
     case F_TAU_X:
       std::copy(data, data + n, h->h_taux.begin());
-      hipLaunchKernelGGL(colphys::k_pack_centre_x, dim3(grid1(ncol, B).x, 1), b, 0, h->stream, h->d_stage, h->d_txc,
+      ++h->tau_gen;
+      hipLaunchKernelGGL(colphys::k_pack_centre_x, colphys::plane_grid(ncol, 1), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, h->d_txc,
                          h->d_col, ncol, P, 1, nx, ny);
       break;
     case F_TAU_Y:
       std::copy(data, data + n, h->h_tauy.begin());
-      hipLaunchKernelGGL(colphys::k_pack_centre_y, dim3(grid1(ncol, B).x, 1), b, 0, h->stream, h->d_stage, h->d_tyc,
+      ++h->tau_gen;
+      hipLaunchKernelGGL(colphys::k_pack_centre_y, colphys::plane_grid(ncol, 1), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, h->d_tyc,
                          h->d_col, ncol, P, 1, nx, ny);
       break;
     default:
@@ -1181,7 +1194,7 @@ int rdb_colphys_get_field(rdb_colphys* h, const char* name, double* out, int n1,
                        ncol);
   } else {
     double* src = layer_ptr(h, name, tracer);
-    hipLaunchKernelGGL(colphys::k_unpack_layer, dim3(grid1(ncol, B).x, e3), dim3(B), 0, h->stream, src, h->d_stage,
+    hipLaunchKernelGGL(colphys::k_unpack_layer, colphys::plane_grid(ncol, e3), dim3(colphys::PLANE_TPB), 0, h->stream, src, h->d_stage,
                        h->d_col, ncol, P, e3, (long long)nx * ny);
   }
   int st = launch_check("unpack");

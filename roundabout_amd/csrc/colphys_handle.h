@@ -62,6 +62,7 @@ struct rdb_colphys {
   unsigned long long* d_acc = nullptr;
   hipStream_t stream = nullptr;
   bool static_dirty = true;
+  bool uv_dirty = false;  // only the centred velocities changed since the last refresh
   std::vector<double> h_u, h_v, h_taux, h_tauy;
   // graph cache
   hipGraph_t graph = nullptr;
@@ -93,6 +94,7 @@ struct rdb_colphys {
   // momentum vertical viscosity: face velocities and fold inputs on the
   // device, created on first use
   colphys::MomState* mom = nullptr;
+  long long tau_gen = 0;  // bumped whenever tau_x or tau_y is set
   long long h_gen = 0;  // bumped whenever h_layer is set (natural-order copies follow it)
   // the rdb_ocean.h host surface: simulation time, and host mirrors of the
   // fields the pointer getters hand out, each current as of state version

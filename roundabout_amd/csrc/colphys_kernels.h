@@ -41,6 +41,13 @@ struct StateView {
   double* pold;     // [2][nz][P] h*c_old of T and S between the two sweeps
 };
 
+// workgroups (of PLANE_TPB threads) of the kernels that move nlev planes of
+// ncol columns between the packed and the full-grid layout
+constexpr int PLANE_TPB = 256;
+inline dim3 plane_grid(int ncol, int nlev) {
+  const unsigned nbx = (unsigned)(ncol + PLANE_TPB - 1) / PLANE_TPB;
+  return dim3(nlev > 1 ? nbx * (unsigned)((nlev + 7) / 8 * 8) : nbx);
+}
 __global__ void k_pack_layer(const double* src, double* dst, const int* col, int ncol, int P, int nlev,
                              long long plane);
 __global__ void k_permute_d(const double* src, double* dst, const int* newpos, int n, int P, int nlev);
@@ -52,6 +59,8 @@ __global__ void k_pack_centre_x(const double* uf, double* dst, const int* col, i
                                 int ny);
 __global__ void k_pack_centre_y(const double* vf, double* dst, const int* col, int ncol, int P, int nlev, int nx,
                                 int ny);
+__global__ void k_pack_centre(const double* uf, const double* vf, double* ub, double* vb, const int* col, int ncol, int P,
+                              int nlev, int nx, int ny);
 __global__ void k_stress_mag(const double* txc, const double* tyc, double* smag, const double* shelf,
                              double* tau_tot, int ncol);
 __global__ void k_cbrt_eval(const double* x, double* y, int n);
@@ -82,7 +91,11 @@ struct SurrView {
   const float* tmax;  // prediction outside it is clamped to it
 };
 
+constexpr int PREP_LEVELS = 8;  // interfaces a lane of k_prepare takes
+__global__ void k_first_live(StateView s, int p0, int p1);
 __global__ void k_prepare(StateView s, Params pr, int p0, int p1);
+template <typename R>
+__global__ void k_dry_columns(StateView s, Params pr, int p0, int p1);
 template <typename R, int NTR, bool TWO_FACTOR, bool SURR>
 __global__ void k_column_step(StateView s, Params pr, double dt, int p0, int p1, unsigned int* guard_count, int M,
                               SurrView sv);
