@@ -21,7 +21,7 @@ LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "librdb_colphys.so"
 
 SOURCES = ["colphys_kernels.hip", "colphys_api.hip", "mlp_kernels.hip", "mlp_net.hip", "mlp_api.hip", "surrogate.hip",
-           "momentum.hip", "boundary.hip", "remap.hip", "contrib.hip"]
+           "momentum.hip", "boundary.hip", "remap.hip", "contrib.hip", "transfer.hip"]
 ARCH = os.environ.get("RDB_COLPHYS_ARCH", "gfx950")
 
 
@@ -59,7 +59,7 @@ def build(verbose: bool = False) -> Path:
         for f in [pool.submit(run, c) for c in cmds]:
             f.result()
     tmp = LIB.with_suffix(".so.tmp")
-    cmd = [cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *objs]
+    cmd = [cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-pthread", "-o", str(tmp), *objs]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)

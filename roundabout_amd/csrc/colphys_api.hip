@@ -53,6 +53,9 @@ int push_error(int status, const char* fmt, ...) {
 
 enum FieldKind { F_LAYER, F_IFACE, F_FACE_X, F_FACE_Y, F_TAU_X, F_TAU_Y, F_COL, F_COL_INT };
 
+// "no offending cell" of scan_h
+const unsigned long long NONE = ~0ull;
+
 struct FieldSpec {
   FieldKind kind;
   bool settable;
@@ -673,6 +676,33 @@ int rdb_colphys_working_precision(void) { return 8; }
 
 namespace {
 
+// New thicknesses in d_stage (the caller's array `data`): the land contract
+// (a dry column holds no live layer, rdb_ocean_state_seed.F90:1842-1880; its
+// outputs are refreshed only when inputs change) and the live levels of every
+// wet column, from the lowest live layer up, for the algorithmic-bytes
+// figure of the step and the autotuner's depth order.
+int scan_h(rdb_colphys* h, const double* data) {
+  const int nx = h->nx, ncol = h->n_all, nz = h->nz;
+  HIP_TRY(hipMemcpyAsync(h->d_acc, &NONE, sizeof NONE, hipMemcpyHostToDevice, h->stream));
+  int* const live = reinterpret_cast<int*>(h->s.fa);
+  hipLaunchKernelGGL(colphys::k_scan_h, grid1(ncol, 256), dim3(256), 0, h->stream, h->d_stage, h->d_col, h->n_wet, ncol,
+                     nz, live, h->d_acc);
+  if (int st = launch_check("k_scan_h")) return st;
+  unsigned long long bad = NONE;
+  HIP_TRY(hipMemcpyAsync(&bad, h->d_acc, sizeof bad, hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  if (bad != NONE) {
+    const int k = (int)(bad / (unsigned long long)ncol), c = (int)(bad % (unsigned long long)ncol);
+    return push_error(RDB_COLPHYS_ERR_CONFIG_VALIDATE,
+                      "set_field h_layer: dry column (i=%d, j=%d) has a live layer k=%d (h=%g > H_VANISHED)", c % nx + 1,
+                      c / nx + 1, k + 1, data[bad]);
+  }
+  h->col_live.resize((size_t)ncol);
+  HIP_TRY(h->xfer->to_host(h->col_live.data(), live, sizeof(int) * (size_t)ncol, h->stream));
+  h->live_levels = std::accumulate(h->col_live.begin(), h->col_live.end(), 0LL);
+  return RDB_COLPHYS_OK;
+}
+
 // One grid's plan: validation, column packing, device buffers.  With a
 // non-null `stream` the plan borrows it (an ensemble member).
 int create_plan(const rdb_colphys_config* cfg, int nx, int ny, int nz, int n_passive, const double* wet,
@@ -696,6 +726,7 @@ int create_plan(const rdb_colphys_config* cfg, int nx, int ny, int nz, int n_pas
     return push_error(RDB_COLPHYS_ERR_SETUP, "create: no HIP device available");
 
   rdb_colphys* h = new rdb_colphys();
+  h->xfer = std::make_shared<colphys::Transfer>();
   h->cfg = *cfg;
   // EPBL and the KPP overlay are mutually exclusive surface schemes: EPBL
   // turns KPP off (rdb_ocean_setup_vmix.F90:697-703)
@@ -926,6 +957,7 @@ int rdb_colphys_ensemble_create(const rdb_colphys_config* cfg, int n_members, co
       break;
     }
     mp->row_off = row;
+    mp->xfer = h->xfer;
     row += mp->n_wet;
     h->members.push_back(mp);
   }
@@ -1048,32 +1080,11 @@ int rdb_colphys_set_field(rdb_colphys* h, const char* name, const double* data, 
     return push_error(RDB_COLPHYS_ERR_BAD_SHAPE, "set_field '%s': shape (%d,%d,%d), expected (%d,%d,%d)", name, n1,
                       n2, n3, e1, e2, e3);
   const size_t n = (size_t)e1 * e2 * e3;
+  HIP_TRY(h->xfer->to_device(h->d_stage, data, 8 * n, h->stream));
   if (!std::strcmp(name, "h_layer")) {
-    // land contract (rdb_ocean_state_seed.F90:1842-1880): a dry column holds
-    // no live layer; its outputs are refreshed only when inputs change.
-    for (int k = 0; k < nz; ++k)
-      for (int c = 0; c < nx * ny; ++c)
-        if (h->dry_host[(size_t)c] && data[(size_t)k * nx * ny + c] > colphys::H_VANISHED)
-          return push_error(RDB_COLPHYS_ERR_CONFIG_VALIDATE,
-                            "set_field h_layer: dry column (i=%d, j=%d) has a live layer k=%d (h=%g > H_VANISHED)",
-                            c % nx + 1, c / nx + 1, k + 1, data[(size_t)k * nx * ny + c]);
-  }
-  if (!std::strcmp(name, "h_layer")) {
-    // live levels per wet column (from the lowest live layer up), for the
-    // algorithmic-bytes figure of the step
-    long long live = 0;
-    h->col_live.assign((size_t)nx * ny, 0);
-    for (int p = 0; p < h->n_wet; ++p) {
-      int c = h->col_host[(size_t)p], kb = nz;
-      for (int k = 0; k < nz; ++k)
-        if (data[(size_t)k * nx * ny + c] > colphys::H_VANISHED) { kb = k; break; }
-      live += nz - kb;
-      h->col_live[(size_t)c] = nz - kb;
-    }
-    h->live_levels = live;
+    if (int st = scan_h(h, data)) return st;
     ++h->h_gen;
   }
-  HIP_TRY(hipMemcpyAsync(h->d_stage, data, 8 * n, hipMemcpyHostToDevice, h->stream));
   const int ncol = h->n_all, P = h->P, B = 256;
   dim3 b(B);
   switch (spec.kind) {
@@ -1091,13 +1102,13 @@ int rdb_colphys_set_field(rdb_colphys* h, const char* name, const double* data, 
       break;
     }
     case F_FACE_X:
-      std::copy(data, data + n, h->h_u.begin());
+      h->xfer->copy(h->h_u.data(), data, 8 * n);
       if (int e = colphys::mom_face_set(h, true)) return e;
       hipLaunchKernelGGL(colphys::k_pack_centre_x, colphys::plane_grid(ncol, nz), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, h->s.ub,
                          h->d_col, ncol, P, nz, nx, ny);
       break;
     case F_FACE_Y:
-      std::copy(data, data + n, h->h_v.begin());
+      h->xfer->copy(h->h_v.data(), data, 8 * n);
       if (int e = colphys::mom_face_set(h, false)) return e;
       hipLaunchKernelGGL(colphys::k_pack_centre_y, colphys::plane_grid(ncol, nz), dim3(colphys::PLANE_TPB), 0, h->stream, h->d_stage, h->s.vb,
                          h->d_col, ncol, P, nz, nx, ny);
@@ -1125,15 +1136,15 @@ int rdb_colphys_set_field(rdb_colphys* h, const char* name, const double* data, 
     st = launch_check("k_stress_mag");
     if (st) return st;
   }
+  // (the caller may reuse its buffer: to_device has read all of it)
   h->static_dirty = true;
-  HIP_TRY(hipStreamSynchronize(h->stream));  // the caller may reuse its buffer
   ++h->state_ver;
   {
     // a host mirror of this field takes the new values directly (as the
     // reference's setters write the host array they push)
     auto it = h->mirrors.find(name);
     if (it != h->mirrors.end() && it->second.size() == n) {
-      std::copy(data, data + n, it->second.begin());
+      h->xfer->copy(it->second.data(), data, 8 * n);
       h->mirror_ver[name] = h->state_ver;
     }
   }
@@ -1176,11 +1187,11 @@ int rdb_colphys_get_field(rdb_colphys* h, const char* name, double* out, int n1,
   switch (spec.kind) {
     case F_FACE_X:
       if (int e = colphys::mom_face_get(h, true)) return e;
-      std::copy(h->h_u.begin(), h->h_u.end(), out);
+      h->xfer->copy(out, h->h_u.data(), 8 * n);
       return RDB_COLPHYS_OK;
     case F_FACE_Y:
       if (int e = colphys::mom_face_get(h, false)) return e;
-      std::copy(h->h_v.begin(), h->h_v.end(), out);
+      h->xfer->copy(out, h->h_v.data(), 8 * n);
       return RDB_COLPHYS_OK;
     case F_TAU_X: std::copy(h->h_taux.begin(), h->h_taux.end(), out); return RDB_COLPHYS_OK;
     case F_TAU_Y: std::copy(h->h_tauy.begin(), h->h_tauy.end(), out); return RDB_COLPHYS_OK;
@@ -1199,8 +1210,7 @@ int rdb_colphys_get_field(rdb_colphys* h, const char* name, double* out, int n1,
   }
   int st = launch_check("unpack");
   if (st) return st;
-  HIP_TRY(hipMemcpyAsync(out, h->d_stage, 8 * n, hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(hipStreamSynchronize(h->stream));
+  HIP_TRY(h->xfer->to_host(out, h->d_stage, 8 * n, h->stream));
   return RDB_COLPHYS_OK;
 }
 

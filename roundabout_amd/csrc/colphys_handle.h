@@ -4,11 +4,13 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
 #include "../../include/rdb_colphys.h"
 #include "colphys_kernels.h"
+#include "transfer.h"
 
 namespace colphys {
 struct SurrState;
@@ -61,6 +63,7 @@ struct rdb_colphys {
   unsigned int* d_guard = nullptr;
   unsigned long long* d_acc = nullptr;
   hipStream_t stream = nullptr;
+  std::shared_ptr<colphys::Transfer> xfer;  // host copies (an ensemble's members share their parent's)
   bool static_dirty = true;
   bool uv_dirty = false;  // only the centred velocities changed since the last refresh
   std::vector<double> h_u, h_v, h_taux, h_tauy;

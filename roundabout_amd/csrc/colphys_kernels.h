@@ -48,6 +48,7 @@ inline dim3 plane_grid(int ncol, int nlev) {
   const unsigned nbx = (unsigned)(ncol + PLANE_TPB - 1) / PLANE_TPB;
   return dim3(nlev > 1 ? nbx * (unsigned)((nlev + 7) / 8 * 8) : nbx);
 }
+__global__ void k_scan_h(const double* h, const int* col, int n_wet, int ncol, int nz, int* live, unsigned long long* bad);
 __global__ void k_pack_layer(const double* src, double* dst, const int* col, int ncol, int P, int nlev,
                              long long plane);
 __global__ void k_permute_d(const double* src, double* dst, const int* newpos, int n, int P, int nlev);

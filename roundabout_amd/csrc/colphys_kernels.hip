@@ -56,6 +56,28 @@ __global__ void k_pack_layer(const double* __restrict__ src, double* __restrict_
   LV(dst, k) = src[(size_t)k * (size_t)plane + (size_t)col[p]];
 }
 
+// New thicknesses in the full-grid layout: live[c] is the number of levels
+// from the lowest live one up of a wet column and 0 of a dry one; *bad takes
+// the lowest cell index (k ncol + c) of a live layer in a dry column.
+// Packed columns [0, n_wet) are the wet ones.
+__global__ void k_scan_h(const double* __restrict__ h, const int* __restrict__ col, int n_wet, int ncol, int nz,
+                         int* __restrict__ live, unsigned long long* bad) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= ncol) return;
+  const int c = col[p];
+  int kb = nz;
+  for (int k0 = 0; k0 < nz && kb == nz; k0 += 8) {
+    double hh[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) hh[q] = h[(size_t)min(k0 + q, nz - 1) * (size_t)ncol + (size_t)c];
+#pragma unroll
+    for (int q = 7; q >= 0; --q)
+      if (k0 + q < nz && hh[q] > H_VANISHED) kb = k0 + q;
+  }
+  live[c] = p < n_wet ? nz - kb : 0;
+  if (p >= n_wet && kb < nz) atomicMin(bad, (unsigned long long)kb * (unsigned long long)ncol + (unsigned long long)c);
+}
+
 // Column repacking for the autotuner: dst[k][newpos[p]] = src[k][p] for the
 // packed columns p < n (the wet ones), nlev levels of pitch P.
 __global__ void k_permute_d(const double* __restrict__ src, double* __restrict__ dst, const int* __restrict__ newpos,

@@ -446,9 +446,8 @@ int mom_ensure(rdb_colphys* h, MomState** out) {
   }
   MomState* m = h->mom;
   if (!m->faces_on_device) {
-    MOM_TRY("face upload", hipMemcpyAsync(m->uf, h->h_u.data(), 8 * h->h_u.size(), hipMemcpyHostToDevice, h->stream));
-    MOM_TRY("face upload", hipMemcpyAsync(m->vf, h->h_v.data(), 8 * h->h_v.size(), hipMemcpyHostToDevice, h->stream));
-    MOM_TRY("face upload", hipStreamSynchronize(h->stream));
+    MOM_TRY("face upload", h->xfer->to_device(m->uf, h->h_u.data(), 8 * h->h_u.size(), h->stream));
+    MOM_TRY("face upload", h->xfer->to_device(m->vf, h->h_v.data(), 8 * h->h_v.size(), h->stream));
     m->faces_on_device = true;
   }
   *out = m;
@@ -463,11 +462,11 @@ void mom_release(rdb_colphys* h) {
 }
 
 int mom_face_set(rdb_colphys* h, bool x_face) {
-  // a new host face field: the device copy follows it
+  // a new host face field, staged in d_stage: the device copy follows it
   MomState* m = h->mom;
   if (!m || !m->faces_on_device) return 0;
   std::vector<double>& src = x_face ? h->h_u : h->h_v;
-  MOM_TRY("face upload", hipMemcpyAsync(x_face ? m->uf : m->vf, src.data(), 8 * src.size(), hipMemcpyHostToDevice,
+  MOM_TRY("face upload", hipMemcpyAsync(x_face ? m->uf : m->vf, h->d_stage, 8 * src.size(), hipMemcpyDeviceToDevice,
                                         h->stream));
   if (x_face)
     m->u_host_stale = false;
@@ -483,9 +482,7 @@ int mom_face_get(rdb_colphys* h, bool x_face) {
   bool& stale = x_face ? m->u_host_stale : m->v_host_stale;
   if (!stale) return 0;
   std::vector<double>& dst = x_face ? h->h_u : h->h_v;
-  MOM_TRY("face download", hipMemcpyAsync(dst.data(), x_face ? m->uf : m->vf, 8 * dst.size(), hipMemcpyDeviceToHost,
-                                          h->stream));
-  MOM_TRY("face download", hipStreamSynchronize(h->stream));
+  MOM_TRY("face download", h->xfer->to_host(dst.data(), x_face ? m->uf : m->vf, 8 * dst.size(), h->stream));
   stale = false;
   return 0;
 }
@@ -513,8 +510,7 @@ int mom_set_field(rdb_colphys* h, const char* name, const double* data, size_t n
     if (st) return st;
     m->fields.push_back({name, d});
   }
-  MOM_TRY("field upload", hipMemcpyAsync(d, data, 8 * n, hipMemcpyHostToDevice, h->stream));
-  MOM_TRY("field upload", hipStreamSynchronize(h->stream));
+  MOM_TRY("field upload", h->xfer->to_device(d, data, 8 * n, h->stream));
   return 0;
 }
 
@@ -534,8 +530,7 @@ int mom_get_field(rdb_colphys* h, const char* name, double* out, size_t n) {
     snprintf(buf, sizeof buf, "get_field '%s': not set (no momentum solve with it yet)", name);
     return rdb_colphys_push_error(RDB_COLPHYS_ERR_NOT_FOUND, buf);
   }
-  MOM_TRY("field download", hipMemcpyAsync(out, d, 8 * n, hipMemcpyDeviceToHost, h->stream));
-  MOM_TRY("field download", hipStreamSynchronize(h->stream));
+  MOM_TRY("field download", h->xfer->to_host(out, d, 8 * n, h->stream));
   return 0;
 }
 
