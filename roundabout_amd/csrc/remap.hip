@@ -274,81 +274,212 @@ struct Win {
   double h, cd, co;
 };
 
-// PQM work arrays, each (nz+1) levels x ncol, level-major.
-enum { P_CD = 0, P_XV, P_C1V, P_XS, P_C1S, P_EVL, P_EVR, P_ESL, P_ESR, P_NARR };
-// The quartic coefficients overwrite arrays that are dead by then.
-enum { P_A = P_XV, P_B = P_C1V, P_C = P_XS, P_D = P_C1S, P_E = P_CD };
+// PQM work arrays, each nz levels x ncol, level-major: the forward sweeps'
+// residuals and scaled super-diagonals of the edge-value and the edge-slope
+// system, which the pass down overwrites with the limited edge values and
+// slopes of each cell.
+enum { P_XV = 0, P_C1V, P_XS, P_C1S, P_NARR };
+enum { P_U0L = P_XV, P_U0R = P_C1V, P_U1L = P_XS, P_U1R = P_C1S };
+
+// Levels of loads in flight ahead of the two PQM passes.
+constexpr int QPF = 4;
+
+// One cell of the W&A limiter, interior (remap_column_pqm :1388-1505).
+__device__ __forceinline__ void pqm_limit(double h_l, double h_c, double h_r, double u_l, double u_c, double u_r,
+                                          double& u0_l, double& u0_r, double& u1_l, double& u1_r) {
+  int infl_l = 0, infl_r = 0;
+  const double sigma_l = 2.0 * (u_c - u_l) / (h_c + NEG);
+  const double sigma_c = 2.0 * (u_r - u_l) / (h_l + 2.0 * h_c + h_r + NEG);
+  const double sigma_r = 2.0 * (u_r - u_c) / (h_c + NEG);
+  double slope;
+  if ((sigma_l * sigma_r) > 0.0)
+    slope = dsign(dmin(dmin(fabs(sigma_l), fabs(sigma_c)), fabs(sigma_r)), sigma_c);
+  else
+    slope = 0.0;
+  if (u1_l * slope <= 0.0) u1_l = slope;
+  if (u1_r * slope <= 0.0) u1_r = slope;
+  if ((u0_r - u_c) * (u_c - u0_l) <= 0.0) {
+    u0_l = u_c;
+    u0_r = u_c;
+    u1_l = 0.0;
+    u1_r = 0.0;
+    infl_l = -1;
+    infl_r = -1;
+  }
+  if (infl_l == 0 && infl_r == 0) {
+    const double b = h_c * u1_l;
+    const double cco = 30.0 * u_c - 12.0 * u0_r - 18.0 * u0_l + 1.5 * h_c * (u1_r - 3.0 * u1_l);
+    const double dco = -60.0 * u_c + h_c * (6.0 * u1_l - 4.0 * u1_r) + 28.0 * u0_r + 32.0 * u0_l;
+    const double eco = 30.0 * u_c + 2.5 * h_c * (u1_r - u1_l) - 15.0 * (u0_l + u0_r);
+    const double alpha1 = 6.0 * eco, alpha2 = 3.0 * dco, alpha3 = cco;
+    const double rho = alpha2 * alpha2 - 4.0 * alpha1 * alpha3;
+    bool flag = false;
+    if ((alpha1 != 0.0) && (rho >= 0.0)) {
+      const double sqrt_rho = sqrt(rho);
+      const double x1 = 0.5 * (-alpha2 - sqrt_rho) / alpha1;
+      const double x2 = 0.5 * (-alpha2 + sqrt_rho) / alpha1;
+      const bool in1 = (x1 >= 0.0) && (x1 <= 1.0), in2 = (x2 >= 0.0) && (x2 <= 1.0);
+      const double g1 = 4.0 * eco * (x1 * x1 * x1) + 3.0 * dco * (x1 * x1) + 2.0 * cco * x1 + b;
+      const double g2 = 4.0 * eco * (x2 * x2 * x2) + 3.0 * dco * (x2 * x2) + 2.0 * cco * x2 + b;
+      if (in1 && in2)
+        flag = (g1 * slope < 0.0) || (g2 * slope < 0.0);
+      else if (in1)
+        flag = g1 * slope < 0.0;
+      else if (in2)
+        flag = g2 * slope < 0.0;
+      if (flag) {
+        if (fabs(sigma_l) < fabs(sigma_r))
+          infl_l = 1;
+        else
+          infl_r = 1;
+      }
+    }
+    if ((alpha1 == 0.0) && (alpha2 != 0.0)) {
+      const double x1 = -alpha3 / alpha2;
+      if ((x1 >= 0.0) && (x1 <= 1.0)) {
+        const double g1 = 4.0 * eco * (x1 * x1 * x1) + 3.0 * dco * (x1 * x1) + 2.0 * cco * x1 + b;
+        if (g1 * slope < 0.0) {
+          if (fabs(sigma_l) < fabs(sigma_r))
+            infl_l = 1;
+          else
+            infl_r = 1;
+        }
+      }
+    }
+  }
+  if (infl_l == 1) {
+    u1_l = (10.0 * u_c - 2.0 * u0_r - 8.0 * u0_l) / (3.0 * h_c + NEG);
+    u1_r = (-10.0 * u_c + 6.0 * u0_r + 4.0 * u0_l) / (h_c + NEG);
+    if (u1_l * slope < 0.0) {
+      u1_l = 0.0;
+      u0_r = 5.0 * u_c - 4.0 * u0_l;
+      u1_r = 20.0 * (u_c - u0_l) / (h_c + NEG);
+    } else if (u1_r * slope < 0.0) {
+      u1_r = 0.0;
+      u0_l = (5.0 * u_c - 3.0 * u0_r) / 2.0;
+      u1_l = 10.0 * (-u_c + u0_r) / (3.0 * h_c + NEG);
+    }
+  } else if (infl_r == 1) {
+    u1_r = (-10.0 * u_c + 8.0 * u0_r + 2.0 * u0_l) / (3.0 * h_c + NEG);
+    u1_l = (10.0 * u_c - 4.0 * u0_r - 6.0 * u0_l) / (h_c + NEG);
+    if (u1_l * slope < 0.0) {
+      u1_l = 0.0;
+      u0_r = (5.0 * u_c - 3.0 * u0_l) / 2.0;
+      u1_r = 10.0 * (u_c - u0_l) / (3.0 * h_c + NEG);
+    } else if (u1_r * slope < 0.0) {
+      u1_r = 0.0;
+      u0_l = 5.0 * u_c - 4.0 * u0_r;
+      u1_l = 20.0 * (-u_c + u0_r) / (h_c + NEG);
+    }
+  }
+}
 
 // ---------------------------------------------------------------------------
-// PQM reconstruction (remap_column_pqm :1226-1539) of one column into the
-// work arrays: the donor column, the two implicit tridiagonal solves for the
-// edge values and slopes, the W&A limiter and the quartic coefficients.
+// PQM reconstruction (remap_column_pqm :1226-1539) of one column: the donor
+// column, the two implicit tridiagonal solves for the edge values and
+// slopes, the limiters.  One pass up (the forward sweeps) and one down: the
+// back substitutions give the edges of cell k from the top, and every later
+// stage looks at most one cell up or down, so bounding (3a), the check of
+// discontinuous edges (3b, pair by pair) and the interior limiter (3c) follow
+// a cell behind in registers.  64 B a cell to the work arrays and 64 B back;
+// in separate passes over nine arrays, a load of each level waited for,
+// 480 x 360 x 75 took 1536 us for a tracer (1119 for a face field), now 422
+// (479), 4 TB/s of work arrays, h and c.
 template <class Cols, bool FIELD>
 __global__ __launch_bounds__(TPB) void k_pqm_coeffs(Cols cols, long ncol, int nz, int be, double* __restrict__ W,
                                                     long arr) {
   const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= ncol) return;
   cols.bind(col);
-  double* const cd = W + P_CD * arr;
   double* const xv = W + P_XV * arr;
   double* const c1v = W + P_C1V * arr;
   double* const xs = W + P_XS * arr;
   double* const c1s = W + P_C1S * arr;
-  double* const evl = W + P_EVL * arr;
-  double* const evr = W + P_EVR * arr;
-  double* const esl = W + P_ESL * arr;
-  double* const esr = W + P_ESR * arr;
 #define AT(a, k) (a)[col + ncol * (long)(k)]
-  // donor-substituted column (rdb_vl_column_conc)
+  // the topmost live layer, the donor of the layers above it
+  int k_top = -1;
+  double c_top = 0.0;
   if (FIELD) {
-    int k_top = -1;
     for (int k = nz - 1; k >= 0; --k)
       if (cols.src_h(k) > HV) {
         k_top = k;
+        c_top = cols.val(k);
         break;
       }
-    if (k_top < 0) {
-      for (int k = 0; k < nz; ++k) AT(cd, k) = 0.0;
-    } else {
-      double cdon = cols.val(k_top);
-      for (int k = nz - 1; k >= 0; --k) {
-        if (cols.src_h(k) > HV) {
-          cdon = cols.val(k);
-          AT(cd, k) = cdon;
-        } else {
-          AT(cd, k) = cdon;
-        }
-      }
+  }
+  struct Cell {
+    double h, q;
+  };
+  auto load = [&](int k) -> Cell { return Cell{cols.src_h(k), cols.val(k)}; };
+  // the donor-substituted value on the way up: the nearest live layer above
+  // (scanned for once a run of fillers), else the topmost live one
+  int la = -1;
+  double la_c = 0.0;
+  auto donor_up = [&](int k, Cell& c) {
+    if (!FIELD || c.h > HV) return;
+    if (k > k_top) {
+      c.q = c_top;  // 0 with no live layer
+      return;
     }
-  } else {
-    for (int k = 0; k < nz; ++k) AT(cd, k) = cols.val(k);
-  }
+    if (la < k) {
+      la = k_top;
+      for (int j0 = k + 1; j0 < k_top && la == k_top; j0 += 8) {
+        double hh[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) hh[u] = cols.src_h(min(j0 + u, k_top));
+#pragma unroll
+        for (int u = 7; u >= 0; --u)
+          if (hh[u] > HV) la = min(j0 + u, k_top);
+      }
+      la_c = cols.val(la);
+    }
+    c.q = la_c;
+  };
   // one-sided four-cell end fits at the bed and (reversed) at the surface
-  double dz4[4], u4[4], bed_v, bed_s, top_v, top_s;
-  for (int m = 0; m < 4; ++m) {
-    dz4[m] = dmax(NEG, cols.src_h(m));
-    u4[m] = AT(cd, m);
+  double bed_v, bed_s, top_v, top_s;
+  {
+    double dz4[4], u4[4];
+    Cell e[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) e[m] = load(m);
+    for (int m = 0; m < 4; ++m) donor_up(m, e[m]);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      dz4[m] = dmax(NEG, e[m].h);
+      u4[m] = e[m].q;
+    }
+    end_value_h4(dz4, u4, bed_v, bed_s);
+    double above = c_top;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) e[m] = load(nz - 1 - m);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (FIELD && !(e[m].h > HV)) e[m].q = above;
+      above = e[m].q;
+      dz4[m] = dmax(NEG, e[m].h);
+      u4[m] = e[m].q;
+    }
+    end_value_h4(dz4, u4, top_v, top_s);
+    la = -1;
   }
-  end_value_h4(dz4, u4, bed_v, bed_s);
-  for (int m = 0; m < 4; ++m) {
-    dz4[m] = dmax(NEG, cols.src_h(nz - 1 - m));
-    u4[m] = AT(cd, nz - 1 - m);
-  }
-  end_value_h4(dz4, u4, top_v, top_s);
   // forward sweep of pqm_solve_diag_dominant for both systems; row 0 is the
   // bed end (diagonal 1, upper 0), rows 1..nz-1 the interior edges
   double d1v = 1.0 * (1.0 / (1.0 + 0.0)), d1s = d1v;
+  double xv_prev, xs_prev;
   {
     const double ip = 1.0 / (1.0 + 0.0);
     AT(c1v, 0) = 0.0 * ip;
     AT(c1s, 0) = 0.0 * ip;
-    AT(xv, 0) = bed_v * ip;
-    AT(xs, 0) = bed_s * ip;
+    xv_prev = bed_v * ip;
+    xs_prev = bed_s * ip;
+    AT(xv, 0) = xv_prev;
+    AT(xs, 0) = xs_prev;
   }
-  double xv_prev = AT(xv, 0), xs_prev = AT(xs, 0);
-  double h_lo = cols.src_h(0), q_lo = AT(cd, 0);
-  for (int k = 1; k <= nz - 1; ++k) {
-    const double h_hi = cols.src_h(k), q_hi = AT(cd, k);
+  Cell lo = load(0);
+  donor_up(0, lo);
+  auto edge_up = [&](int k, Cell hi) {
+    donor_up(k, hi);
+    const double h_lo = lo.h, h_hi = hi.h, q_lo = lo.q, q_hi = hi.q;
     // edge values (:1266-1281)
     {
       double h0 = dmax(h_lo, NEG);
@@ -390,181 +521,128 @@ __global__ __launch_bounds__(TPB) void k_pqm_coeffs(Cols cols, long ncol, int nz
       xs_prev = (r - al * xs_prev) * ip;
       AT(xs, k) = xs_prev;
     }
-    h_lo = h_hi;
-    q_lo = q_hi;
+    lo = hi;
+  };
+  {
+    Cell ring[QPF];
+#pragma unroll
+    for (int j = 0; j < QPF; ++j) ring[j] = load(min(1 + j, nz - 1));
+    for (int k0 = 1; k0 <= nz - 1; k0 += QPF) {
+#pragma unroll
+      for (int j = 0; j < QPF; ++j) {
+        const Cell cur = ring[j];
+        ring[j] = load(min(k0 + j + QPF, nz - 1));
+        if (k0 + j <= nz - 1) edge_up(k0 + j, cur);
+      }
+    }
   }
   // last row: the surface end (lower 0, diagonal 1), then back-substitution
   {
     const double ipv = 1.0 / (1.0 + d1v * 0.0);
     xv_prev = (top_v - 0.0 * xv_prev) * ipv;
-    AT(xv, nz) = xv_prev;
     const double ips = 1.0 / (1.0 + d1s * 0.0);
     xs_prev = (-top_s - 0.0 * xs_prev) * ips;
-    AT(xs, nz) = xs_prev;
   }
-  for (int k = nz - 1; k >= 0; --k) {
-    xv_prev = AT(xv, k) - AT(c1v, k) * xv_prev;
-    AT(xv, k) = xv_prev;
-    xs_prev = AT(xs, k) - AT(c1s, k) * xs_prev;
-    AT(xs, k) = xs_prev;
-  }
-  // 3a. bound_edge_values (:1346-1370)
-  for (int k = 0; k < nz; ++k) {
-    const int kl = k > 0 ? k - 1 : 0, kr = k < nz - 1 ? k + 1 : nz - 1;
-    const double u_l = AT(cd, kl), u_c = AT(cd, k), u_r = AT(cd, kr);
-    const double h_l = cols.src_h(kl), h_c = cols.src_h(k), h_r = cols.src_h(kr);
-    double ev_l = AT(xv, k), ev_r = AT(xv, k + 1);
-    double slope_x_h = 0.0;
-    if (((h_l + h_r) + 2.0 * h_c) > 0.0) {
-      const double sigma_l = (u_c - u_l);
-      const double sigma_c = (u_r - u_l) * (h_c / ((h_l + h_r) + 2.0 * h_c));
-      const double sigma_r = (u_r - u_c);
-      if ((sigma_l * sigma_r) > 0.0) slope_x_h = dsign(dmin(dmin(fabs(sigma_l), fabs(sigma_c)), fabs(sigma_r)), sigma_c);
-    }
-    if ((u_l - ev_l) * (ev_l - u_c) < 0.0) ev_l = u_c - dsign(dmin(fabs(slope_x_h), fabs(ev_l - u_c)), slope_x_h);
-    if ((u_r - ev_r) * (ev_r - u_c) < 0.0) ev_r = u_c + dsign(dmin(fabs(slope_x_h), fabs(ev_r - u_c)), slope_x_h);
-    ev_l = dmax(dmin(ev_l, dmax(u_l, u_c)), dmin(u_l, u_c));
-    ev_r = dmax(dmin(ev_r, dmax(u_r, u_c)), dmin(u_r, u_c));
-    AT(evl, k) = ev_l;
-    AT(evr, k) = ev_r;
-    AT(esl, k) = AT(xs, k);
-    AT(esr, k) = AT(xs, k + 1);
-  }
-  // 3b. check_discontinuous_edge_values (:1375-1384)
-  for (int k = 0; k < nz - 1; ++k) {
-    const double qa = AT(cd, k), qb = AT(cd, k + 1);
-    const double er = AT(evr, k), el = AT(evl, k + 1);
-    if ((el - er) * (qb - qa) < 0.0) {
-      double u0_avg = 0.5 * (er + el);
-      u0_avg = dmax(dmin(u0_avg, dmax(qa, qb)), dmin(qa, qb));
-      AT(evr, k) = u0_avg;
-      AT(evl, k + 1) = u0_avg;
-    }
-  }
-  // 3c. interior cells (:1388-1505)
-  for (int k = 1; k <= nz - 2; ++k) {
-    int infl_l = 0, infl_r = 0;
-    double u0_l = AT(evl, k), u0_r = AT(evr, k);
-    double u1_l = AT(esl, k), u1_r = AT(esr, k);
-    const double h_l = cols.src_h(k - 1), h_c = cols.src_h(k), h_r = cols.src_h(k + 1);
-    const double u_l = AT(cd, k - 1), u_c = AT(cd, k), u_r = AT(cd, k + 1);
-    const double sigma_l = 2.0 * (u_c - u_l) / (h_c + NEG);
-    const double sigma_c = 2.0 * (u_r - u_l) / (h_l + 2.0 * h_c + h_r + NEG);
-    const double sigma_r = 2.0 * (u_r - u_c) / (h_c + NEG);
-    double slope;
-    if ((sigma_l * sigma_r) > 0.0)
-      slope = dsign(dmin(dmin(fabs(sigma_l), fabs(sigma_c)), fabs(sigma_r)), sigma_c);
-    else
-      slope = 0.0;
-    if (u1_l * slope <= 0.0) u1_l = slope;
-    if (u1_r * slope <= 0.0) u1_r = slope;
-    if ((u0_r - u_c) * (u_c - u0_l) <= 0.0) {
-      u0_l = u_c;
-      u0_r = u_c;
-      u1_l = 0.0;
-      u1_r = 0.0;
-      infl_l = -1;
-      infl_r = -1;
-    }
-    if (infl_l == 0 && infl_r == 0) {
-      const double b = h_c * u1_l;
-      const double cco = 30.0 * u_c - 12.0 * u0_r - 18.0 * u0_l + 1.5 * h_c * (u1_r - 3.0 * u1_l);
-      const double dco = -60.0 * u_c + h_c * (6.0 * u1_l - 4.0 * u1_r) + 28.0 * u0_r + 32.0 * u0_l;
-      const double eco = 30.0 * u_c + 2.5 * h_c * (u1_r - u1_l) - 15.0 * (u0_l + u0_r);
-      const double alpha1 = 6.0 * eco, alpha2 = 3.0 * dco, alpha3 = cco;
-      const double rho = alpha2 * alpha2 - 4.0 * alpha1 * alpha3;
-      bool flag = false;
-      if ((alpha1 != 0.0) && (rho >= 0.0)) {
-        const double sqrt_rho = sqrt(rho);
-        const double x1 = 0.5 * (-alpha2 - sqrt_rho) / alpha1;
-        const double x2 = 0.5 * (-alpha2 + sqrt_rho) / alpha1;
-        const bool in1 = (x1 >= 0.0) && (x1 <= 1.0), in2 = (x2 >= 0.0) && (x2 <= 1.0);
-        const double g1 = 4.0 * eco * (x1 * x1 * x1) + 3.0 * dco * (x1 * x1) + 2.0 * cco * x1 + b;
-        const double g2 = 4.0 * eco * (x2 * x2 * x2) + 3.0 * dco * (x2 * x2) + 2.0 * cco * x2 + b;
-        if (in1 && in2)
-          flag = (g1 * slope < 0.0) || (g2 * slope < 0.0);
-        else if (in1)
-          flag = g1 * slope < 0.0;
-        else if (in2)
-          flag = g2 * slope < 0.0;
-        if (flag) {
-          if (fabs(sigma_l) < fabs(sigma_r))
-            infl_l = 1;
-          else
-            infl_r = 1;
-        }
-      }
-      if ((alpha1 == 0.0) && (alpha2 != 0.0)) {
-        const double x1 = -alpha3 / alpha2;
-        if ((x1 >= 0.0) && (x1 <= 1.0)) {
-          const double g1 = 4.0 * eco * (x1 * x1 * x1) + 3.0 * dco * (x1 * x1) + 2.0 * cco * x1 + b;
-          if (g1 * slope < 0.0) {
-            if (fabs(sigma_l) < fabs(sigma_r))
-              infl_l = 1;
-            else
-              infl_r = 1;
-          }
-        }
-      }
-    }
-    if (infl_l == 1) {
-      u1_l = (10.0 * u_c - 2.0 * u0_r - 8.0 * u0_l) / (3.0 * h_c + NEG);
-      u1_r = (-10.0 * u_c + 6.0 * u0_r + 4.0 * u0_l) / (h_c + NEG);
-      if (u1_l * slope < 0.0) {
-        u1_l = 0.0;
-        u0_r = 5.0 * u_c - 4.0 * u0_l;
-        u1_r = 20.0 * (u_c - u0_l) / (h_c + NEG);
-      } else if (u1_r * slope < 0.0) {
-        u1_r = 0.0;
-        u0_l = (5.0 * u_c - 3.0 * u0_r) / 2.0;
-        u1_l = 10.0 * (-u_c + u0_r) / (3.0 * h_c + NEG);
-      }
-    } else if (infl_r == 1) {
-      u1_r = (-10.0 * u_c + 8.0 * u0_r + 2.0 * u0_l) / (3.0 * h_c + NEG);
-      u1_l = (10.0 * u_c - 4.0 * u0_r - 6.0 * u0_l) / (h_c + NEG);
-      if (u1_l * slope < 0.0) {
-        u1_l = 0.0;
-        u0_r = (5.0 * u_c - 3.0 * u0_l) / 2.0;
-        u1_r = 10.0 * (u_c - u0_l) / (3.0 * h_c + NEG);
-      } else if (u1_r * slope < 0.0) {
-        u1_r = 0.0;
-        u0_l = 5.0 * u_c - 4.0 * u0_r;
-        u1_l = 20.0 * (-u_c + u0_r) / (h_c + NEG);
-      }
-    }
-    AT(evl, k) = u0_l;
-    AT(evr, k) = u0_r;
-    AT(esl, k) = u1_l;
-    AT(esr, k) = u1_r;
-  }
-  // boundary cells (:1507-1532), then the quartic of every cell (:1535-1549);
-  // the last coefficient overwrites the donor column, so the mean below is
-  // carried in a register
-  double u_below = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    const double h_c = cols.src_h(k), u_c = AT(cd, k);
-    double u0_l = AT(evl, k), u0_r = AT(evr, k), u1_l = AT(esl, k), u1_r = AT(esr, k);
+  struct Row {
+    double xv, c1v, xs, c1s, h, q;  // rows k of the systems, cell k - 1
+  };
+  auto load_row = [&](int k) -> Row {
+    const int kk = max(k, 0), kc = max(k - 1, 0);
+    return Row{AT(xv, kk), AT(c1v, kk), AT(xs, kk), AT(c1s, kk), cols.src_h(kc), cols.val(kc)};
+  };
+  // cells k + 2, k + 1, k and k - 1 (the end cell again past an end), and the
+  // bounded edges and slopes of cell k + 1, whose upper pair is settled
+  Cell c2{0.0, 0.0}, c1, c0;
+  double el1 = 0.0, er1 = 0.0, sl1 = 0.0, sr1 = 0.0;
+  double above = c_top;
+  c0 = load(nz - 1);
+  if (FIELD && !(c0.h > HV)) c0.q = above;
+  above = c0.q;
+  c1 = c0;
+  // the finished cell k: the end cells (:1507-1532) or the interior limiter
+  auto finish = [&](int k, Cell dn, Cell c, Cell up, double u0_l, double u0_r, double u1_l, double u1_r) {
     if (k == 0 || k == nz - 1) {
-      u0_l = u_c;
-      u0_r = u_c;
+      u0_l = c.q;
+      u0_r = c.q;
       u1_l = 0.0;
       u1_r = 0.0;
       if (be) {
-        const double d = (k == 0) ? half_jump(h_c, cols.src_h(1), AT(cd, 1) - u_c)
-                                  : half_jump(h_c, cols.src_h(nz - 2), u_c - u_below);
-        u0_l = u_c - d;
-        u0_r = u_c + d;
-        u1_l = 2.0 * d / dmax(h_c, NEG);
+        const double d = (k == 0) ? half_jump(c.h, up.h, up.q - c.q) : half_jump(c.h, dn.h, c.q - dn.q);
+        u0_l = c.q - d;
+        u0_r = c.q + d;
+        u1_l = 2.0 * d / dmax(c.h, NEG);
         u1_r = u1_l;
       }
+    } else {
+      pqm_limit(dn.h, c.h, up.h, dn.q, c.q, up.q, u0_l, u0_r, u1_l, u1_r);
     }
-    AT(W + P_A * arr, k) = u0_l;
-    AT(W + P_B * arr, k) = h_c * u1_l;
-    AT(W + P_C * arr, k) = 30.0 * u_c - 12.0 * u0_r - 18.0 * u0_l + 1.5 * h_c * (u1_r - 3.0 * u1_l);
-    AT(W + P_D * arr, k) = -60.0 * u_c + h_c * (6.0 * u1_l - 4.0 * u1_r) + 28.0 * u0_r + 32.0 * u0_l;
-    AT(W + P_E * arr, k) = 30.0 * u_c + 2.5 * h_c * (u1_r - u1_l) - 15.0 * (u0_l + u0_r);
-    u_below = u_c;
+    AT(W + P_U0L * arr, k) = u0_l;
+    AT(W + P_U0R * arr, k) = u0_r;
+    AT(W + P_U1L * arr, k) = u1_l;
+    AT(W + P_U1R * arr, k) = u1_r;
+  };
+  auto cell_down = [&](int k, const Row& r) {
+    const double ev_r0 = xv_prev, es_r0 = xs_prev;
+    xv_prev = r.xv - r.c1v * xv_prev;
+    xs_prev = r.xs - r.c1s * xs_prev;
+    Cell dn = c0;
+    if (k > 0) {
+      dn = Cell{r.h, r.q};
+      if (FIELD && !(dn.h > HV)) dn.q = above;
+      above = dn.q;
+    }
+    // 3a. bound_edge_values (:1346-1370)
+    double el = xv_prev, er = ev_r0;
+    {
+      const double u_l = dn.q, u_c = c0.q, u_r = c1.q;
+      const double h_l = dn.h, h_c = c0.h, h_r = c1.h;
+      double slope_x_h = 0.0;
+      if (((h_l + h_r) + 2.0 * h_c) > 0.0) {
+        const double sigma_l = (u_c - u_l);
+        const double sigma_c = (u_r - u_l) * (h_c / ((h_l + h_r) + 2.0 * h_c));
+        const double sigma_r = (u_r - u_c);
+        if ((sigma_l * sigma_r) > 0.0)
+          slope_x_h = dsign(dmin(dmin(fabs(sigma_l), fabs(sigma_c)), fabs(sigma_r)), sigma_c);
+      }
+      if ((u_l - el) * (el - u_c) < 0.0) el = u_c - dsign(dmin(fabs(slope_x_h), fabs(el - u_c)), slope_x_h);
+      if ((u_r - er) * (er - u_c) < 0.0) er = u_c + dsign(dmin(fabs(slope_x_h), fabs(er - u_c)), slope_x_h);
+      el = dmax(dmin(el, dmax(u_l, u_c)), dmin(u_l, u_c));
+      er = dmax(dmin(er, dmax(u_r, u_c)), dmin(u_r, u_c));
+    }
+    if (k < nz - 1) {
+      // 3b. check_discontinuous_edge_values (:1375-1384) of cells k, k + 1
+      const double qa = c0.q, qb = c1.q;
+      if ((el1 - er) * (qb - qa) < 0.0) {
+        double u0_avg = 0.5 * (er + el1);
+        u0_avg = dmax(dmin(u0_avg, dmax(qa, qb)), dmin(qa, qb));
+        er = u0_avg;
+        el1 = u0_avg;
+      }
+      finish(k + 1, c0, c1, c2, el1, er1, sl1, sr1);
+    }
+    el1 = el;
+    er1 = er;
+    sl1 = xs_prev;
+    sr1 = es_r0;
+    c2 = c1;
+    c1 = c0;
+    c0 = dn;
+  };
+  {
+    Row ring[QPF];
+#pragma unroll
+    for (int j = 0; j < QPF; ++j) ring[j] = load_row(nz - 1 - j);
+    for (int k0 = nz - 1; k0 >= 0; k0 -= QPF) {
+#pragma unroll
+      for (int j = 0; j < QPF; ++j) {
+        if (k0 - j >= 0) {
+          cell_down(k0 - j, ring[j]);
+          ring[j] = load_row(k0 - j - QPF);
+        }
+      }
+    }
   }
+  finish(0, c1, c1, c2, el1, er1, sl1, sr1);
 #undef AT
 }
 
@@ -722,12 +800,16 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
       rb = qR;
       r6 = q6;
     } else if (M == M_PQM) {
+      // the quartic of the cell's edge values and slopes (:1535-1549)
       const long at = col + ncol * (long)s;
-      ra = W[P_A * arr + at];
-      rb = W[P_B * arr + at];
-      r6 = W[P_C * arr + at];
-      rd = W[P_D * arr + at];
-      re = W[P_E * arr + at];
+      const double u0_l = W[P_U0L * arr + at], u0_r = W[P_U0R * arr + at];
+      const double u1_l = W[P_U1L * arr + at], u1_r = W[P_U1R * arr + at];
+      const double u_c = w1.cd, h_c = w1.h;
+      ra = u0_l;
+      rb = h_c * u1_l;
+      r6 = 30.0 * u_c - 12.0 * u0_r - 18.0 * u0_l + 1.5 * h_c * (u1_r - 3.0 * u1_l);
+      rd = -60.0 * u_c + h_c * (6.0 * u1_l - 4.0 * u1_r) + 28.0 * u0_r + 32.0 * u0_l;
+      re = 30.0 * u_c + 2.5 * h_c * (u1_r - u1_l) - 15.0 * (u0_l + u0_r);
     }
   };
   auto advance = [&]() {
@@ -1043,7 +1125,7 @@ int launch(const Cols& cols, long ncol, int nz, int method, int be, int nu, doub
   double* W = nullptr;
   long arr = 0;
   if (m == M_PQM) {
-    arr = (long)(nz + 1) * ncol;
+    arr = (long)nz * ncol;
     void* p = nullptr;
     int rc = ensure(g_pqm, sizeof(double) * (size_t)arr * P_NARR, &p);
     if (rc) return rc;
