@@ -650,14 +650,37 @@ __global__ __launch_bounds__(TPB) void k_pqm_coeffs(Cols cols, long ncol, int nz
 // The merge walk.  FIELD: the concentration-form tracer pipeline of
 // ocean_remap_tracer_field (donor column, filler excess, bounding, budget);
 // otherwise the plain remap_column of the face and raw-column passes.
-template <class Cols, int M, bool FIELD>
-__global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int be, int nu,
-                                              const double* __restrict__ W, long arr, double* __restrict__ out,
-                                              double* __restrict__ budget, double* __restrict__ clamp) {
+//
+// What bounds it is issue: on 1440 x 1080 x 75 (PPM, tracers and faces) 508
+// vector instructions a level and wavefront before the kept quotient and the
+// shared way on to the next cell, 442 now, the vector pipes busy two thirds of
+// the time; 2.50 -> 2.26 ms a tracer, and 0.35 ms of copy-back gone in place.
+// (Levels in blocks through LDS, one round trip for four of them, cost more
+// instructions than the latency they hid: 2.6 ms.)
+//
+// In place (scratch given: cols' field is out itself) target k may be
+// written once level k has gone through the window (k <= s + 2): everything
+// read later lies above.  A lane whose targets run ahead of its sources
+// further than that writes to scratch from there on and copies those levels
+// at its end; the excesses of a target with more than two filler
+// contributors, which are otherwise gathered from the field again, go to the
+// second half of scratch.
+//
+// A batch too small to fill the chip is split (SPLIT) over gridDim.y lanes a
+// column, each with a run of the targets: such a lane adds up the thicknesses below
+// (the same running sums) to where its targets begin, and starts the walk one
+// source cell early for the edge that the first one takes over.  Not in
+// place: other lanes' targets are this one's sources.
+template <class Cols, int M, bool FIELD, bool SPLIT>
+__global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, int be, int nu,
+                                              const double* __restrict__ W, long arr, double* out,
+                                              double* __restrict__ budget, double* __restrict__ clamp,
+                                              double* __restrict__ scratch) {
   const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= ncol) return;
   cols.bind(col);
 
+  const long arr2 = ncol * (long)nz;  // the second half of scratch
   // Source cells arrive through a two-deep prefetch of their raw (h, c)
   // (loaded two advances before the window takes them), so the load
   // latency overlaps the reconstruction of the cells in between.
@@ -695,6 +718,15 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
         }
         // the nearest live layer above; none above: the topmost live one
         // (the last live layer loaded); no live layer: 0
+        if (SPLIT && la >= nz && !have_live && blockIdx.y > 0) {
+          // none above, and the walk began above the topmost live layer
+          for (int j = m - 1; j >= 0 && !have_live; --j)
+            if (cols.src_h(j) > HV) {
+              last_live = cols.val(j);
+              have_live = true;
+            }
+          have_live = true;  // (0 with no live layer)
+        }
         w.cd = (la < nz) ? la_c : (have_live ? last_live : 0.0);
       }
     }
@@ -709,17 +741,59 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
     return 0.0;
   };
 
+  // this lane's targets [k0, k1)
+  const int k0 = SPLIT ? (int)((long)nz * blockIdx.y / gridDim.y) : 0;
+  const int k1 = SPLIT ? (int)((long)nz * (blockIdx.y + 1) / gridDim.y) : nz;
+  double zn_hi = 0.0;
+  int s = 0, s_first_cell = 0;  // the first cell walked, and the one where the targets begin
+  double zs_lo = 0.0;
+  if (SPLIT && k0 > 0) {
+    for (int j0 = 0; j0 < k0; j0 += 8) {
+      double h[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) h[u] = cols.dst_h(min(j0 + u, nz - 1));
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (j0 + u < k0) zn_hi = zn_hi + h[u];
+    }
+    // the first source cell whose top lies above, and the bottom of the one below it
+    double z = 0.0, z_below = 0.0;
+    bool found = false;
+    for (int j0 = 0; j0 < nz && !found; j0 += 8) {
+      double h[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) h[u] = cols.src_h(min(j0 + u, nz - 1));
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (!found && j0 + u < nz) {
+          const double top = z + h[u];
+          if (top <= zn_hi) {
+            s_first_cell = j0 + u + 1;
+            z_below = z;
+            z = top;
+          } else {
+            found = true;
+          }
+        }
+    }
+    s = s_first_cell > 0 ? s_first_cell - 1 : 0;
+    zs_lo = s_first_cell > 0 ? z_below : 0.0;
+  }
   Win w0{0.0, 0.0, 0.0};
-  Win w1 = finish(0, raw(0));
-  Win w2 = finish(1, raw(1));
-  Win w3 = finish(2, raw(2));
-  Raw pa = raw(3), pb = raw(4);
+  if (SPLIT && s > 0) w0 = finish(s - 1, raw(s - 1));
+  Win w1 = finish(s, raw(s));
+  Win w2 = finish(s + 1, raw(s + 1));
+  Win w3 = finish(s + 2, raw(s + 2));
+  Raw pa = raw(s + 3), pb = raw(s + 4);
   const double cd0 = w1.cd;
-  int s = 0;
-  double zs_lo = 0.0, zs_hi = 0.0 + w1.h;
+  double zs_hi = zs_lo + w1.h;
   // reconstruction of cell s: PLM slope in ra; PPM/H4 (q_L, q_R, q6) in
   // (ra, rb, r6); PQM coefficients in (ra, rb, r6, rd, re)
   double ra = 0.0, rb = 0.0, r6 = 0.0, rd = 0.0, re = 0.0, carry = 0.0;
+  // the position in cell s where the last overlap with it ended, and the
+  // next begins: the quotient of the same operands, kept
+  double x_end = 0.0;
+  bool x_kept = false;
 
   auto recon = [&]() {
     if (M == M_PLM) {
@@ -822,14 +896,16 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
     pb = raw(s + 4);
     zs_lo = zs_hi;
     zs_hi = zs_lo + w1.h;
+    x_kept = false;
     if (s < nz) recon();
   };
   recon();
+  if (SPLIT && s < s_first_cell) advance();
 
   // target thicknesses arrive two targets ahead
-  double hn_a = cols.dst_h(0), hn_b = (nz > 1) ? cols.dst_h(1) : 0.0;
-  double zn_hi = 0.0;
-  for (int k = 0; k < nz; ++k) {
+  double hn_a = cols.dst_h(k0), hn_b = (k0 + 1 < nz) ? cols.dst_h(k0 + 1) : 0.0;
+  int defer = nz;  // in place: targets from here on are in scratch
+  for (int k = k0; k < k1; ++k) {
     const double hn = hn_a;
     hn_a = hn_b;
     hn_b = (k + 2 < nz) ? cols.dst_h(k + 2) : 0.0;
@@ -854,17 +930,23 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
         const double z_hi = dmin(zn_hi, zs_hi);
         const double ov = z_hi - z_lo;
         if (ov > 0.0) {
+          // the cell's local coordinates of the overlap's ends; at its own
+          // bottom 0 / h = 0
+          double xl = 0.0, xh = 0.0;
+          if (M != M_PCM) {
+            if (z_lo != zs_lo) xl = x_kept ? x_end : (z_lo - zs_lo) / w1.h;
+            xh = (z_hi - zs_lo) / w1.h;
+            x_end = xh;
+            x_kept = true;
+          }
           if (M == M_PCM) {
             integral = integral + w1.cd * ov;
           } else if (M == M_PLM) {
-            const double xl = (z_lo - zs_lo) / w1.h, xh = (z_hi - zs_lo) / w1.h;
             integral = integral + ov * (w1.cd + ra * (xl + xh - 1.0));
           } else if (M == M_PPM || M == M_H4) {
-            const double xl = (z_lo - zs_lo) / w1.h, xh = (z_hi - zs_lo) / w1.h;
             integral = integral + w1.h * ((xh - xl) * ra + 0.5 * (xh * xh - xl * xl) * (rb - ra + r6) -
                                           (xh * xh * xh - xl * xl * xl) * r6 / 3.0);
           } else if (M == M_PQM) {
-            const double xl = (z_lo - zs_lo) / w1.h, xh = (z_hi - zs_lo) / w1.h;
             integral = integral + ov * (ra + rb * 0.5 * (xl + xh) + r6 * (1.0 / 3.0) * (xl * xl + xh * xh + xl * xh) +
                                         rd * 0.25 * ((xl * xl + xh * xh) * (xl + xh)) +
                                         re * 0.2 * ((xh * xh * xh + xl * xl * xl) * (xl + xh) + xl * xl * xh * xh));
@@ -894,6 +976,8 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
                   ex0 = sx * ov;
                 else if (n_ex == 1)
                   ex1 = sx * ov;
+                else if (scratch)
+                  scratch[arr2 + col + ncol * (long)(n_ex - 2)] = sx * ov;
                 ++n_ex;
               }
             }
@@ -907,8 +991,12 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
           }
           ++n_hit;
         }
-        if (!(zs_hi < zn_hi) || s + 1 >= nz) break;
+        // a source cell that ends with the target is left here as well, so
+        // that the loop above the targets (the same code again) hardly runs
+        const bool more = zs_hi < zn_hi;
+        if (!(zs_hi <= zn_hi) || s + 1 >= nz) break;
         advance();
+        if (!more) break;
       }
     }
     double q;
@@ -916,15 +1004,19 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
       q = cd0;
     else
       q = (hn > 0.0) ? integral / hn : 0.0;
+    // in place: is level k still to be read?
+    if (scratch && defer == nz && k > s + 2) defer = k;
+    double* const to = (scratch && k >= defer) ? scratch : out;
     if (!FIELD) {
-      __builtin_nontemporal_store(q, &out[at]);
+      __builtin_nontemporal_store(q, &to[at]);
       continue;
     }
     // remap_add_filler_excess: each filler contributor's own excess, after
     // the division, in source order
-    if (n_ex <= 2) {
+    if (n_ex <= 2 || scratch) {
       if (n_ex > 0) q = q + ex0 / hn;
       if (n_ex > 1) q = q + ex1 / hn;
+      for (int j = 2; j < n_ex; ++j) q = q + scratch[arr2 + col + ncol * (long)(j - 2)] / hn;
     } else {
       double zj_lo = z_first;
       for (int j = s_first; j <= s; ++j) {
@@ -946,7 +1038,6 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
       cn = isfinite(c_raw) ? dmax(c_lo, dmin(c_hi, c_raw)) : c_raw;
     else
       cn = fallback;
-    __builtin_nontemporal_store(cn, &out[at]);
     if (clamp) clamp[at] = hn * (cn - c_raw);
     if (budget) {
       // the source cell of level k: from the window when it is there
@@ -972,25 +1063,49 @@ __global__ __launch_bounds__(TPB) void k_walk(Cols cols, long ncol, int nz, int 
       const double p_old = h_k * c_k;
       budget[at] = b_old + (p_new - p_old);
     }
+    __builtin_nontemporal_store(cn, &to[at]);  // after the read of its own source cell
   }
+  if (scratch)
+    for (int k = defer; k < nz; ++k) {
+      const long at = col + ncol * (long)k;
+      out[at] = scratch[at];
+    }
 }
 
 // rescale_anomaly_ke (rdb_ocean_remap.F90:1131-1180) of a remapped face
 // column: u holds u_old on entry and the result on exit, un the remap.
+// (480 x 360 x 75: 300 -> 258 us, 4 TB/s over its three passes)
+constexpr int KEL = 6;
 __global__ __launch_bounds__(TPB) void k_face_ke(FaceCols cols, long ncol, int nz, const double* __restrict__ un,
                                                  double* __restrict__ u) {
   const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= ncol) return;
   cols.bind(col);
   double h_old_sum = 0.0, h_new_sum = 0.0, mom_old = 0.0, mom_new = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    double o, n;
-    cols.pair(k, o, n);
-    const long at = col + ncol * (long)k;
-    h_old_sum = h_old_sum + o;
-    h_new_sum = h_new_sum + n;
-    mom_old = mom_old + o * u[at];
-    mom_new = mom_new + n * un[at];
+  // the sums are serial, their loads are not: KEL levels a round
+  struct Level {
+    double o, n, u, un;
+  };
+  auto load = [&](int k0, Level (&q)[KEL]) {
+#pragma unroll
+    for (int j = 0; j < KEL; ++j) {
+      const int k = min(k0 + j, nz - 1);
+      cols.pair(k, q[j].o, q[j].n);
+      q[j].u = u[col + ncol * (long)k];
+      q[j].un = un[col + ncol * (long)k];
+    }
+  };
+  for (int k0 = 0; k0 < nz; k0 += KEL) {
+    Level q[KEL];
+    load(k0, q);
+#pragma unroll
+    for (int j = 0; j < KEL; ++j)
+      if (k0 + j < nz) {
+        h_old_sum = h_old_sum + q[j].o;
+        h_new_sum = h_new_sum + q[j].n;
+        mom_old = mom_old + q[j].o * q[j].u;
+        mom_new = mom_new + q[j].n * q[j].un;
+      }
   }
   double scale_fac = -1.0;  // < 0: leave the remap as it is
   double u_bar_new = 0.0;
@@ -998,14 +1113,17 @@ __global__ __launch_bounds__(TPB) void k_face_ke(FaceCols cols, long ncol, int n
     const double u_bar_old = mom_old / h_old_sum;
     u_bar_new = mom_new / h_new_sum;
     double ke_old = 0.0, ke_new = 0.0;
-    for (int k = 0; k < nz; ++k) {
-      double o, n;
-      cols.pair(k, o, n);
-      const long at = col + ncol * (long)k;
-      double anom = u[at] - u_bar_old;
-      ke_old = ke_old + 0.5 * o * anom * anom;
-      anom = un[at] - u_bar_new;
-      ke_new = ke_new + 0.5 * n * anom * anom;
+    for (int k0 = 0; k0 < nz; k0 += KEL) {
+      Level q[KEL];
+      load(k0, q);
+#pragma unroll
+      for (int j = 0; j < KEL; ++j)
+        if (k0 + j < nz) {
+          double anom = q[j].u - u_bar_old;
+          ke_old = ke_old + 0.5 * q[j].o * anom * anom;
+          anom = q[j].un - u_bar_new;
+          ke_new = ke_new + 0.5 * q[j].n * anom * anom;
+        }
     }
     if (!(ke_new <= 0.0 || ke_old <= 0.0)) {
       scale_fac = sqrt(ke_old / ke_new);
@@ -1013,9 +1131,14 @@ __global__ __launch_bounds__(TPB) void k_face_ke(FaceCols cols, long ncol, int n
       if (scale_fac < 0.0) scale_fac = 0.0;
     }
   }
-  for (int k = 0; k < nz; ++k) {
-    const long at = col + ncol * (long)k;
-    u[at] = (scale_fac >= 0.0) ? u_bar_new + scale_fac * (un[at] - u_bar_new) : un[at];
+  for (int k0 = 0; k0 < nz; k0 += KEL) {
+    double q[KEL];
+#pragma unroll
+    for (int j = 0; j < KEL; ++j) q[j] = un[col + ncol * (long)min(k0 + j, nz - 1)];
+#pragma unroll
+    for (int j = 0; j < KEL; ++j)
+      if (k0 + j < nz)
+        u[col + ncol * (long)(k0 + j)] = (scale_fac >= 0.0) ? u_bar_new + scale_fac * (q[j] - u_bar_new) : q[j];
   }
 }
 
@@ -1111,6 +1234,14 @@ int effective_method(int method, int nz) {
   return m;
 }
 
+// Lanes a column of the walk: one where the columns alone put two wavefronts
+// on every SIMD (256 CUs of four; 131 072 columns), else as many as do, of at
+// least four targets each (1000 columns x 33, PPM_H4: 80 us, 20 split).
+int walk_splits(long ncol, int nz) {
+  const long want = 131072 / ncol;
+  return (int)(want < 1 ? 1 : want > nz / 4 ? (nz / 4 > 1 ? nz / 4 : 1) : want);
+}
+
 bool overlaps(const void* a, const void* b, size_t bytes) {
   const char* x = static_cast<const char*>(a);
   const char* y = static_cast<const char*>(b);
@@ -1119,9 +1250,12 @@ bool overlaps(const void* a, const void* b, size_t bytes) {
 
 template <class Cols, bool FIELD>
 int launch(const Cols& cols, long ncol, int nz, int method, int be, int nu, double* out, double* budget,
-           double* clamp, hipStream_t st) {
+           double* clamp, double* scratch, hipStream_t st) {
   const int m = effective_method(method, nz);
   const unsigned grid = (unsigned)((ncol + TPB - 1) / TPB);
+  // (small batches in workgroups of one wavefront, over more CUs)
+  const unsigned splits = scratch ? 1u : (unsigned)walk_splits(ncol, nz);
+  const unsigned wtpb = splits > 1 ? 64u : (unsigned)TPB, wgrid = (unsigned)((ncol + wtpb - 1) / wtpb);
   double* W = nullptr;
   long arr = 0;
   if (m == M_PQM) {
@@ -1135,8 +1269,9 @@ int launch(const Cols& cols, long ncol, int nz, int method, int be, int nu, doub
   switch (m) {
 #define RDB_REMAP_CASE(MM)                                                                                        \
   case MM:                                                                                                        \
-    hipLaunchKernelGGL((k_walk<Cols, MM, FIELD>), dim3(grid), dim3(TPB), 0, st, cols, ncol, nz, be, nu, W, arr, out, \
-                       budget, clamp);                                                                            \
+    hipLaunchKernelGGL((splits > 1 ? k_walk<Cols, MM, FIELD, true> : k_walk<Cols, MM, FIELD, false>), \
+                       dim3(wgrid, splits), dim3(wtpb), 0, st, cols, ncol, nz, be, nu, W, arr, out, \
+                       budget, clamp, scratch);                                                                            \
     break;
     RDB_REMAP_CASE(M_PCM)
     RDB_REMAP_CASE(M_PLM)
@@ -1172,19 +1307,21 @@ int rdb_remap_tracer_field(int method, int nx, int ny, int nz, const double* h_o
   const long ncol = (long)nx * ny;
   const size_t bytes = sizeof(double) * (size_t)ncol * nz;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  double* out = c_out;
-  const bool in_place = overlaps(c_in, c_out, bytes);
-  if (in_place) {
+  // in place: the walk's own rules; other overlaps through a buffer
+  double *out = c_out, *scratch = nullptr;
+  const bool in_place = c_in == c_out && walk_splits(ncol, nz) == 1;
+  const bool through = !in_place && overlaps(c_in, c_out, bytes);
+  if (in_place || through) {
     void* p = nullptr;
-    int rc = ensure(g_out, bytes, &p);
+    int rc = ensure(g_out, in_place ? 2 * bytes : bytes, &p);
     if (rc) return rc;
-    out = static_cast<double*>(p);
+    (in_place ? scratch : out) = static_cast<double*>(p);
   }
   CellCols cols{h_old, h_new, c_in, ncol, 0};
   int rc = launch<CellCols, true>(cols, ncol, nz, method, bnd_extrap ? 1 : 0, nonunif ? 1 : 0, out, budget,
-                                  clamp_out, st);
+                                  clamp_out, scratch, st);
   if (rc) return rc;
-  if (in_place) {
+  if (through) {
     const hipError_t e = hipMemcpyAsync(c_out, out, bytes, hipMemcpyDeviceToDevice, st);
     if (e != hipSuccess) return fail(RDB_COLPHYS_ERR_SETUP, "remap_tracer_field: copy-back", e);
   }
@@ -1201,18 +1338,23 @@ int rdb_remap_face_velocity(int axis, int nx, int ny, int nz, const double* h_ol
   const long ncol = nfu * nfv;
   const size_t bytes = sizeof(double) * (size_t)ncol * nz;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // the KE rescale reads the old field and the remapped one; without it a
+  // walk of one lane a column runs in place
   void* p = nullptr;
-  int rc = ensure(g_out, bytes, &p);
+  const bool in_place = !conserve_ke && walk_splits(ncol, nz) == 1;
+  int rc = ensure(g_out, in_place ? 2 * bytes : bytes, &p);
   if (rc) return rc;
-  double* un = static_cast<double*>(p);
+  double* const buf = static_cast<double*>(p);
+  double* const un = in_place ? u : buf;
   FaceCols cols{h_old, h_new, u, (long)nx * ny, ncol, nx, ny, axis, zlevel_faces ? 1 : 0, 0, 0, 0, 0};
-  rc = launch<FaceCols, false>(cols, ncol, nz, method, bnd_extrap ? 1 : 0, nonunif ? 1 : 0, un, nullptr, nullptr, st);
+  rc = launch<FaceCols, false>(cols, ncol, nz, method, bnd_extrap ? 1 : 0, nonunif ? 1 : 0, un, nullptr, nullptr,
+                               in_place ? buf : nullptr, st);
   if (rc) return rc;
   if (conserve_ke) {
     hipLaunchKernelGGL(k_face_ke, dim3((unsigned)((ncol + TPB - 1) / TPB)), dim3(TPB), 0, st, cols, ncol, nz, un, u);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(RDB_COLPHYS_ERR_SETUP, "remap_face_velocity: KE rescale launch", e);
-  } else {
+  } else if (!in_place) {
     const hipError_t e = hipMemcpyAsync(u, un, bytes, hipMemcpyDeviceToDevice, st);
     if (e != hipSuccess) return fail(RDB_COLPHYS_ERR_SETUP, "remap_face_velocity: copy-back", e);
   }
@@ -1226,19 +1368,20 @@ int rdb_remap_columns(int method, int ncol, int nz, const double* dz_old, const 
     return rdb_colphys_push_error(RDB_COLPHYS_ERR_BAD_SHAPE, "remap_columns: NULL");
   const size_t bytes = sizeof(double) * (size_t)ncol * nz;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  double* out = q_new;
-  const bool in_place = overlaps(q_old, q_new, bytes);
-  if (in_place) {
+  double *out = q_new, *scratch = nullptr;
+  const bool in_place = q_old == q_new && walk_splits(ncol, nz) == 1;
+  const bool through = !in_place && overlaps(q_old, q_new, bytes);
+  if (in_place || through) {
     void* p = nullptr;
-    int rc = ensure(g_out, bytes, &p);
+    int rc = ensure(g_out, in_place ? 2 * bytes : bytes, &p);
     if (rc) return rc;
-    out = static_cast<double*>(p);
+    (in_place ? scratch : out) = static_cast<double*>(p);
   }
   CellCols cols{dz_old, dz_new, q_old, (long)ncol, 0};
   int rc = launch<CellCols, false>(cols, ncol, nz, method, bnd_extrap ? 1 : 0, nonunif ? 1 : 0, out, nullptr,
-                                   nullptr, st);
+                                   nullptr, scratch, st);
   if (rc) return rc;
-  if (in_place) {
+  if (through) {
     const hipError_t e = hipMemcpyAsync(q_new, out, bytes, hipMemcpyDeviceToDevice, st);
     if (e != hipSuccess) return fail(RDB_COLPHYS_ERR_SETUP, "remap_columns: copy-back", e);
   }

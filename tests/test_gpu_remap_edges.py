@@ -44,3 +44,69 @@ def test_pqm_layer_counts(orc, nz):
         d_u = R.DeviceArray.from_host(u)
         R.ocean_apply_ale_remap_faces(d_ho, d_hn, d_u, None, 5, conserve_ke=be, zlevel_faces=nu, bnd_extrap=be, nonunif=nu)
         assert np.array_equal(d_u.to_host(), orc.remap_face_velocity(0, ho, hn, u, 5, be, nu, be, nu))
+
+
+def _tiled(ho, hn, c, nx, ny):
+    """The field repeated to (nx, ny): enough columns for one lane each."""
+    reps = (-(-nx // ho.shape[0]), -(-ny // ho.shape[1]), 1)
+    return [np.asfortranarray(np.tile(a, reps)[:nx, :ny]) for a in (ho, hn, c)]
+
+
+def _far_targets(ho, hn, rng):
+    """Targets that run ahead of their sources (thin ones over a thick bed
+    cell) and behind, and targets over three and more stale fillers."""
+    nx, ny, nz = ho.shape
+    for i in range(0, nx, 3):
+        for j in range(0, ny, 2):
+            kind = (i // 3 + j) % 4
+            if kind == 0:
+                ho[i, j, 0] = 40.0 * nz
+                hn[i, j, :-1] = 0.5 + rng.random(nz - 1)
+            elif kind == 1:
+                hn[i, j, 0] = 40.0 * nz
+                ho[i, j, :-1] = 0.5 + rng.random(nz - 1)
+            elif kind == 2 and nz > 6:
+                ho[i, j, 1:6] = 1.0e-4
+                hn[i, j, :3] = 0.2
+            elif kind == 3 and nz > 6:
+                ho[i, j, -6:-1] = 7.0e-5
+                hn[i, j, -2:] = 3.0
+            total = ho[i, j].sum()
+            hn[i, j, -1] = 0.0
+            if hn[i, j].sum() > total:
+                hn[i, j] *= 0.9 * total / hn[i, j].sum()
+            hn[i, j, -1] = total - hn[i, j, :-1].sum()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(31, 20, 3), (31, 20, 8), (31, 20, 33), (270, 250, 3), (270, 250, 9), (262, 251, 17)])
+@pytest.mark.parametrize("method", [1, 2, 3, 4, 5])
+def test_in_place_and_split_walks(orc, nx, ny, nz, method):
+    """Below 65 537 columns a column's targets are split over lanes, above one
+    lane walks them, in place without a buffer: both, in place and out of
+    place, on targets ahead of and behind their sources."""
+    rng = np.random.default_rng(nz)
+    ho, hn, c = _field(31, 20, nz, 90 + nz)
+    _far_targets(ho, hn, rng)
+    be, nu = method % 2, nz % 2
+    print(f"[case] walk {nx}x{ny}x{nz} method={method} be={be} nu={nu}", flush=True)
+    bud = np.zeros_like(ho, order="F")
+    want, want_cl = orc.remap_tracer_field(method, ho, hn, c, be, nu, budget=bud)
+    want, want_cl, bud = _tiled(want, want_cl, bud, nx, ny)
+    ho, hn, c = _tiled(ho, hn, c, nx, ny)
+    d_ho, d_hn = R.DeviceArray.from_host(ho), R.DeviceArray.from_host(hn)
+    for in_place in (True, False):
+        d_c, d_b, d_cl = R.DeviceArray.from_host(c), R.DeviceArray.zeros(c.shape), R.DeviceArray(c.shape)
+        d_o = None if in_place else R.DeviceArray(c.shape)
+        out = R.ocean_remap_tracer_field(d_ho, d_hn, d_c, method, bnd_extrap=be, nonunif=nu, budget=d_b, clamp_out=d_cl,
+                                         c_out=d_o)
+        for name, g, w in (("c", out, want), ("budget", d_b, bud), ("clamp", d_cl, want_cl)):
+            assert np.array_equal(g.to_host(), w), (name, in_place)
+    u = np.asfortranarray(rng.normal(0, 0.2, (nx + 1, ny, nz)))
+    d_u = R.DeviceArray.from_host(u)
+    R.ocean_apply_ale_remap_faces(d_ho, d_hn, d_u, None, method, bnd_extrap=be, nonunif=nu)
+    assert np.array_equal(d_u.to_host(), orc.remap_face_velocity(0, ho, hn, u, method, 0, 0, be, nu))
+    d_q = R.DeviceArray.from_host(c.reshape(-1, nz, order="F"))
+    cols = [R.DeviceArray.from_host(a.reshape(-1, nz, order="F")) for a in (ho, hn)]
+    got = R.remap_column(*cols, d_q, method, bnd_extrap=be, nonunif=nu).to_host()
+    R.remap_column(*cols, d_q, method, bnd_extrap=be, nonunif=nu, q_new=d_q)
+    assert np.array_equal(d_q.to_host(), got)
