@@ -703,6 +703,28 @@ int scan_h(rdb_colphys* h, const double* data) {
   return RDB_COLPHYS_OK;
 }
 
+// The launch shape of the fused step before any tuning.  Up to eight
+// wavefronts a CU (what its registers hold) the wet columns go out in
+// workgroups of one wavefront, so that they spread over all CUs, beyond that
+// in workgroups of 256; the LDS of a CU is shared out to its wavefronts for
+// the Thomas state, up to max_levels levels.  us a step, a workgroup of 256
+// with nothing in LDS -> this rule: 3 624 columns of 20 levels 41.9 -> 40.1,
+// 14 336 of 75 139.6 -> 125.6, 30 240 155.2 -> 134.1, 53 760 161.7 -> 154.0,
+// 120 960 214.2 -> 200.0, 336 000 of 60 389.4 -> 363.1 (with 64 threads there
+// 376.0).  An ensemble's persistent launch wants no more than eight levels
+// (six members, 65 965 columns: 148.0 -> 131.8; 152.7 with 16).
+void default_shape(rdb_colphys* h, long long columns, int nz, int max_levels) {
+  if (h->block_pinned) return;
+  int dev = 0, n_cu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cu < 1)
+    return;
+  const long long per_cu = std::max((columns + 64LL * n_cu - 1) / (64LL * n_cu), 1LL);
+  const long long nq = 3 + std::min(h->n_passive, 4) + (h->cfg.kt_bg != h->cfg.ks_bg ? 1 : 0);
+  h->block = per_cu <= 8 ? 64 : 256;
+  h->lds_levels = (int)std::min<long long>(std::min(nz, max_levels), h->lds_max / (std::min(per_cu, 8LL) * 64 * nq * 8));
+}
+
 // One grid's plan: validation, column packing, device buffers.  With a
 // non-null `stream` the plan borrows it (an ensemble member).
 int create_plan(const rdb_colphys_config* cfg, int nx, int ny, int nz, int n_passive, const double* wet,
@@ -800,6 +822,7 @@ int create_plan(const rdb_colphys_config* cfg, int nx, int ny, int nz, int n_pas
     h->order_mode = 1;
   }
   h->n_wet = (int)wet_idx.size();
+  default_shape(h, h->n_wet, nz, 32);
   h->n_all = ncol;
   h->P = ((ncol + 63) / 64) * 64;
   h->col_host = wet_idx;
@@ -968,6 +991,7 @@ int rdb_colphys_ensemble_create(const rdb_colphys_config* cfg, int n_members, co
   // single-grid code path that reaches it touches nothing
   h->nz_net = nz_max;
   h->ens_wet = row;
+  default_shape(h, row, nz_max, 8);
   if (!st && row > 0x7fffffffLL) st = push_error(RDB_COLPHYS_ERR_BAD_SHAPE, "ensemble_create: too many wet columns");
   if (!st) {
     const size_t nm = h->members.size();
