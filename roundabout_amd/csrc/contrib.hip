@@ -535,7 +535,7 @@ constexpr int BED_WAVES = 8;
 // per column: a serial chain of about 550 vector instructions an interface,
 // 2 us of it at one or two wavefronts a SIMD, so the longest chain bounds the
 // kernel.  On 480 x 360 x 75 (121 000 wet columns) one solve took 1.66 ms,
-// eight sweeps of 74 interfaces in the columns over fillers; now 0.22 ms here
+// eight sweeps of 74 interfaces in the columns over fillers; now 0.22-0.27 ms here
 // and 0.49 ms in k_epbl_bed.  What gave it: those columns' sweeps side by
 // side; the last guess's sweep carried on where it stopped instead of
 // repeated; one evaluation of v* and K an interface; levels through LDS.
