@@ -331,7 +331,9 @@ __global__ void __launch_bounds__(MTPB) k_vdiff_momentum(MomView vu, MomView vv,
     double c, d, g;
   };
   auto load_b = [&](int k, Back& q) {
-    const int kk = max(k, k_lo);  // (k_lo <= nz - 1: stored above)
+    // (row nz - 1 exists also where k_lo lies above it: k_bot and k_top both
+    // beyond nz leave every row the identity, and the loops below are empty)
+    const int kk = min(max(k, k_lo), nz - 1);
     q.c = v.cd[f + F * kk];
     if (fl.solve) q.d = v.rd[f + F * kk];
     if (fl.remnant) q.g = v.rem[f + F * kk];

@@ -153,3 +153,27 @@ def test_column_step_reads_the_new_velocities(orc):
                            ("v_face_y_layer", v)):
             got = cp.get_field(name)
             assert np.array_equal(got, want), (name, int(np.sum(got != want)))
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(9, 7, 1), (33, 18, 6), (40, 25, 7), (64, 64, 20)])
+@pytest.mark.parametrize("remnant_only", [False, True])
+def test_bottom_and_top_rows_beyond_the_column(orc, nx, ny, nz, remnant_only):
+    """Faces whose k_bot and k_top both lie above nz (no row to solve), next
+    to faces with one of them there: identity columns, as the oracle's."""
+    print(f"[case] momentum, k_bot/k_top beyond nz, {nx}x{ny}x{nz} remnant_only={remnant_only}", flush=True)
+    ocean = synth.make_ocean(nx, ny, nz, 8, land_frac=0.2, topo="zstar")
+    rng = np.random.default_rng(nz)
+    f = {}
+    for tag, shp in (("u", (nx + 1, ny)), ("v", (nx, ny + 1))):
+        for end in ("k_bot", "k_top"):
+            beyond = nz + rng.integers(1, 300, shp)
+            f[f"{end}_{tag}"] = np.where(rng.random(shp) < 0.5, beyond, rng.integers(1, nz + 1, shp)).astype(float)
+    kw = dict(implicit_stress=True, remnant=True, remnant_only=remnant_only, K_v_momentum=1e-2)
+    u, v, ru, rv = orc.vdiff_apply_momentum(ocean.h, ocean.u, ocean.v, ocean.wet, DT, tau_u=ocean.tau_x,
+                                            tau_v=ocean.tau_y, rho0=default_config().rho0, **f, **kw)
+    with ColumnPhysics.from_ocean(ocean) as cp:
+        for name, arr in f.items():
+            cp.set_field(name, arr)
+        cp.vdiff_momentum(DT, use_kv_source=0, **{k: (int(x) if isinstance(x, bool) else x) for k, x in kw.items()})
+        for name, want in (("u_face_x_layer", u), ("v_face_y_layer", v), ("visc_rem_u", ru), ("visc_rem_v", rv)):
+            assert np.array_equal(cp.get_field(name), want), name
