@@ -791,7 +791,8 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
   // (ra, rb, r6); PQM coefficients in (ra, rb, r6, rd, re)
   double ra = 0.0, rb = 0.0, r6 = 0.0, rd = 0.0, re = 0.0, carry = 0.0;
   // the position in cell s where the last overlap with it ended, and the
-  // next begins: the quotient of the same operands, kept
+  // next begins: the quotient of the same operands, kept (not across a target
+  // of no or negative thickness, which may move the next one's bottom back)
   double x_end = 0.0;
   bool x_kept = false;
 
@@ -913,6 +914,7 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
     const double b_old = (FIELD && budget) ? budget[at] : 0.0;
     const double zn_lo = zn_hi;
     zn_hi = zn_lo + hn;
+    if (!(hn > 0.0)) x_kept = false;
     // the first source cell whose top lies above the target's bottom
     while (s < nz && zs_hi <= zn_lo) advance();
     const double fallback = (s < nz) ? w1.co : w0.co;  // c_own(min(ko0, nz))

@@ -110,3 +110,21 @@ def test_in_place_and_split_walks(orc, nx, ny, nz, method):
     got = R.remap_column(*cols, d_q, method, bnd_extrap=be, nonunif=nu).to_host()
     R.remap_column(*cols, d_q, method, bnd_extrap=be, nonunif=nu, q_new=d_q)
     assert np.array_equal(d_q.to_host(), got)
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(31, 20, 3), (31, 20, 33), (270, 250, 9)])
+@pytest.mark.parametrize("method", [1, 2, 3, 4, 5])
+def test_round_off_negative_targets(orc, nx, ny, nz, method):
+    """Targets a round-off below zero, as a difference of interfaces leaves
+    them: the next target begins a little below where the last one ended."""
+    print(f"[case] negative targets {nx}x{ny}x{nz} method={method}", flush=True)
+    rng = np.random.default_rng(7 * nz)
+    ho = 1.0 + 25.0 * rng.random((31, 20, nz))
+    hn = ho * (0.4 + 1.2 * rng.random((31, 20, nz)))
+    c = 30.0 + 5.0 * rng.random((31, 20, nz))
+    hn[rng.random((31, 20, nz)) < 0.15] = -1.0e-15
+    want, _ = orc.remap_tracer_field(method, ho, hn, c, 0, 0)
+    want, ho, hn, c = _tiled(want, ho, c, nx, ny)[:1] + _tiled(ho, hn, c, nx, ny)
+    d = [R.DeviceArray.from_host(a) for a in (ho, hn, c)]
+    R.ocean_remap_tracer_field(*d, method)
+    assert np.array_equal(d[2].to_host(), want)
