@@ -748,33 +748,53 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
   int s = 0, s_first_cell = 0;  // the first cell walked, and the one where the targets begin
   double zs_lo = 0.0;
   if (SPLIT && k0 > 0) {
+    bool rising = true;  // the targets' interfaces
     for (int j0 = 0; j0 < k0; j0 += 8) {
       double h[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) h[u] = cols.dst_h(min(j0 + u, nz - 1));
 #pragma unroll
       for (int u = 0; u < 8; ++u)
-        if (j0 + u < k0) zn_hi = zn_hi + h[u];
-    }
-    // the first source cell whose top lies above, and the bottom of the one below it
-    double z = 0.0, z_below = 0.0;
-    bool found = false;
-    for (int j0 = 0; j0 < nz && !found; j0 += 8) {
-      double h[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) h[u] = cols.src_h(min(j0 + u, nz - 1));
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (!found && j0 + u < nz) {
-          const double top = z + h[u];
-          if (top <= zn_hi) {
-            s_first_cell = j0 + u + 1;
-            z_below = z;
-            z = top;
-          } else {
-            found = true;
-          }
+        if (j0 + u < k0) {
+          zn_hi = zn_hi + h[u];
+          rising = rising && h[u] >= 0.0;
         }
+    }
+    double z = 0.0, z_below = 0.0;
+    if (rising) {
+      // the first source cell whose top lies above, and the bottom of the one below it
+      bool found = false;
+      for (int j0 = 0; j0 < nz && !found; j0 += 8) {
+        double h[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) h[u] = cols.src_h(min(j0 + u, nz - 1));
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (!found && j0 + u < nz) {
+            const double top = z + h[u];
+            if (top <= zn_hi) {
+              s_first_cell = j0 + u + 1;
+              z_below = z;
+              z = top;
+            } else {
+              found = true;
+            }
+          }
+      }
+    } else {
+      // a negative or NaN target below: the cells that one lane would have
+      // passed on its way here
+      double zn = 0.0;
+      for (int j = 0; j <= k0; ++j) {
+        while (s_first_cell < nz) {
+          const double top = z + cols.src_h(s_first_cell);
+          if (!(top <= zn)) break;
+          ++s_first_cell;
+          z_below = z;
+          z = top;
+        }
+        if (j < k0) zn = zn + cols.dst_h(j);
+      }
     }
     s = s_first_cell > 0 ? s_first_cell - 1 : 0;
     zs_lo = s_first_cell > 0 ? z_below : 0.0;

@@ -128,3 +128,28 @@ def test_round_off_negative_targets(orc, nx, ny, nz, method):
     d = [R.DeviceArray.from_host(a) for a in (ho, hn, c)]
     R.ocean_remap_tracer_field(*d, method)
     assert np.array_equal(d[2].to_host(), want)
+
+
+@pytest.mark.parametrize("kind", ["negative", "nan", "negative source"])
+@pytest.mark.parametrize("nz", [8, 33, 75])
+def test_split_lanes_start_where_one_lane_would(nz, kind):
+    """Thicknesses outside the stated range give what one lane a column gives
+    (the same columns in a batch of more than 65 536)."""
+    rng = np.random.default_rng(nz)
+    ho = 1.0 + 25.0 * rng.random((31, 20, nz))
+    hn = ho * (0.4 + 1.2 * rng.random((31, 20, nz)))
+    c = 30.0 + 5.0 * rng.random((31, 20, nz))
+    some = rng.random((31, 20, nz)) < 0.1
+    if kind == "nan":
+        hn[some & (rng.random(some.shape) < 0.4)] = np.nan
+    else:
+        a = hn if kind == "negative" else ho
+        a[some] *= -rng.random(int(some.sum()))
+    for method in (1, 2, 3, 4, 5):
+        print(f"[case] {kind} nz={nz} method={method}", flush=True)
+        got = []
+        for shape in ((31, 20), (270, 250)):
+            d = [R.DeviceArray.from_host(a) for a in _tiled(ho, hn, c, *shape)]
+            R.ocean_remap_tracer_field(*d, method)
+            got.append(d[2].to_host()[:31, :20])
+        assert np.array_equal(*got, equal_nan=True), method
