@@ -662,9 +662,11 @@ __global__ __launch_bounds__(TPB) void k_pqm_coeffs(Cols cols, long ncol, int nz
 // written once level k has gone through the window (k <= s + 2): everything
 // read later lies above.  A lane whose targets run ahead of its sources
 // further than that writes to scratch from there on and copies those levels
-// at its end; the excesses of a target with more than two filler
-// contributors, which are otherwise gathered from the field again, go to the
-// second half of scratch.
+// at its end.  The excesses of a target with more than two filler
+// contributors, which are otherwise gathered from the field again, go to
+// scratch as well, from level 0 up: the j-th of them comes with a source cell
+// s >= j, so a deferred target that it displaces has its level behind the
+// window and is written out first.  One field of scratch serves both.
 //
 // A batch too small to fill the chip is split (SPLIT) over gridDim.y lanes a
 // column, each with a run of the targets: such a lane adds up the thicknesses below
@@ -680,7 +682,6 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
   if (col >= ncol) return;
   cols.bind(col);
 
-  const long arr2 = ncol * (long)nz;  // the second half of scratch
   // Source cells arrive through a two-deep prefetch of their raw (h, c)
   // (loaded two advances before the window takes them), so the load
   // latency overlaps the reconstruction of the cells in between.
@@ -925,7 +926,7 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
 
   // target thicknesses arrive two targets ahead
   double hn_a = cols.dst_h(k0), hn_b = (k0 + 1 < nz) ? cols.dst_h(k0 + 1) : 0.0;
-  int defer = nz;  // in place: targets from here on are in scratch
+  int defer = nz;  // in place: targets from here up to the current one are in scratch
   for (int k = k0; k < k1; ++k) {
     const double hn = hn_a;
     hn_a = hn_b;
@@ -998,8 +999,15 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
                   ex0 = sx * ov;
                 else if (n_ex == 1)
                   ex1 = sx * ov;
-                else if (scratch)
-                  scratch[arr2 + col + ncol * (long)(n_ex - 2)] = sx * ov;
+                else if (scratch) {
+                  const int j = n_ex - 2;
+                  const long to = col + ncol * (long)j;
+                  if (j >= defer && j < k) {  // (j == defer: the ones below went first)
+                    out[to] = scratch[to];
+                    defer = j + 1;
+                  }
+                  scratch[to] = sx * ov;
+                }
                 ++n_ex;
               }
             }
@@ -1038,7 +1046,7 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
     if (n_ex <= 2 || scratch) {
       if (n_ex > 0) q = q + ex0 / hn;
       if (n_ex > 1) q = q + ex1 / hn;
-      for (int j = 2; j < n_ex; ++j) q = q + scratch[arr2 + col + ncol * (long)(j - 2)] / hn;
+      for (int j = 2; j < n_ex; ++j) q = q + scratch[col + ncol * (long)(j - 2)] / hn;
     } else {
       double zj_lo = z_first;
       for (int j = s_first; j <= s; ++j) {
@@ -1335,7 +1343,7 @@ int rdb_remap_tracer_field(int method, int nx, int ny, int nz, const double* h_o
   const bool through = !in_place && overlaps(c_in, c_out, bytes);
   if (in_place || through) {
     void* p = nullptr;
-    int rc = ensure(g_out, in_place ? 2 * bytes : bytes, &p);
+    int rc = ensure(g_out, bytes, &p);
     if (rc) return rc;
     (in_place ? scratch : out) = static_cast<double*>(p);
   }
@@ -1364,7 +1372,7 @@ int rdb_remap_face_velocity(int axis, int nx, int ny, int nz, const double* h_ol
   // walk of one lane a column runs in place
   void* p = nullptr;
   const bool in_place = !conserve_ke && walk_splits(ncol, nz) == 1;
-  int rc = ensure(g_out, in_place ? 2 * bytes : bytes, &p);
+  int rc = ensure(g_out, bytes, &p);
   if (rc) return rc;
   double* const buf = static_cast<double*>(p);
   double* const un = in_place ? u : buf;
@@ -1395,7 +1403,7 @@ int rdb_remap_columns(int method, int ncol, int nz, const double* dz_old, const 
   const bool through = !in_place && overlaps(q_old, q_new, bytes);
   if (in_place || through) {
     void* p = nullptr;
-    int rc = ensure(g_out, in_place ? 2 * bytes : bytes, &p);
+    int rc = ensure(g_out, bytes, &p);
     if (rc) return rc;
     (in_place ? scratch : out) = static_cast<double*>(p);
   }

@@ -4,6 +4,8 @@ columns and targets far from their sources, against the oracle, bitwise."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -153,3 +155,58 @@ def test_split_lanes_start_where_one_lane_would(nz, kind):
             R.ocean_remap_tracer_field(*d, method)
             got.append(d[2].to_host()[:31, :20])
         assert np.array_equal(*got, equal_nan=True), method
+
+
+@pytest.mark.parametrize("nz", [7, 12, 24])
+@pytest.mark.parametrize("method", [1, 3, 5])
+def test_deferred_targets_and_many_excesses(orc, nz, method):
+    """Thin targets far ahead of their sources, then one over a long run of
+    stale fillers, in place: its excesses lie in scratch where the deferred
+    targets wait."""
+    rng = np.random.default_rng(nz)
+    ho = 2.0 + 20.0 * rng.random((31, 20, nz))
+    c = 30.0 + 5.0 * rng.random((31, 20, nz))
+    hn = np.empty_like(ho)
+    for i in range(31):
+        for j in range(20):
+            bed, thin = int(rng.integers(1, 3)), int(rng.integers(0, nz - 2))
+            fill = int(rng.integers(2, max(3, nz - 1 - bed)))
+            ho[i, j, :bed] = 100.0
+            ho[i, j, bed:bed + fill] = 2.0e-5 + 1.2e-4 * rng.random(fill)
+            total = ho[i, j].sum()
+            hn[i, j, :thin] = 90.0 * bed / nz * rng.random(thin)
+            rest = rng.random(nz - thin)
+            rest[0] += 3.0
+            hn[i, j, thin:] = rest * (total - hn[i, j, :thin].sum()) / rest.sum()
+    bud = np.zeros_like(ho, order="F")
+    print(f"[case] deferred targets and excesses nz={nz} method={method}", flush=True)
+    want, want_cl = orc.remap_tracer_field(method, ho, hn, c, 0, 0, budget=bud)
+    want, want_cl, bud = _tiled(want, want_cl, bud, 270, 250)
+    ho, hn, c = _tiled(ho, hn, c, 270, 250)
+    d_ho, d_hn, d_c = (R.DeviceArray.from_host(a) for a in (ho, hn, c))
+    d_b, d_cl = R.DeviceArray.zeros(c.shape), R.DeviceArray(c.shape)
+    R.ocean_remap_tracer_field(d_ho, d_hn, d_c, method, budget=d_b, clamp_out=d_cl)
+    for name, g, w in (("c", d_c, want), ("budget", d_b, bud), ("clamp", d_cl, want_cl)):
+        assert np.array_equal(g.to_host(), w), name
+
+
+def test_in_place_calls_hold_one_field_of_scratch():
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert R._hip().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    print("[case] scratch of in-place calls, 128 MiB fields", flush=True)
+    h = R.DeviceArray.from_host(np.full((65536, 256), 10.0, order="F"))
+    q = h.copy()
+    R.remap_column(h, h, q, 1, q_new=q)  # lanes share a column: through a buffer of one field
+    R.synchronize()
+    before = free()
+    for a in (h, q):
+        a.shape = (131072, 128)
+    R.remap_column(h, h, q, 1, q_new=q)  # one lane a column
+    for a in (h, q):
+        a.shape = (512, 256, 128)
+    R.ocean_remap_tracer_field(h, h, q, 1)
+    R.synchronize()
+    assert before - free() < 64 << 20
