@@ -34,7 +34,7 @@ struct MomFlags {
 
 struct MomView {
   int nu, nv, nz, nx, ny, x_face;
-  double* u;           // [nz][nu * nv]
+  double* u;           // [nz][nu * nv]; holds the Thomas d' between the two sweeps
   const double* h;     // [nz][nx * ny]
   const double* kv;    // [nz + 1][nx * ny] (unused with scalar_kv)
   const double* wet;   // [nx * ny]
@@ -48,7 +48,6 @@ struct MomView {
   const double* ktop;  // 1-based layer index, or null: nz
   const double* kbot;  // 1-based layer index, or null: 1
   double* cd;          // Thomas c' [nz][nu * nv]
-  double* rd;          // Thomas d'
   double* rem;         // visc_rem
 };
 
@@ -311,7 +310,7 @@ __global__ void __launch_bounds__(MTPB) k_vdiff_momentum(MomView vu, MomView vv,
     // leaves u as it is, the remnant is 1)
     if (k >= k_lo) {
       v.cd[f + F * k] = cp;
-      if (fl.solve) v.rd[f + F * k] = dp;
+      if (fl.solve) v.u[f + F * k] = dp;  // (this level's u went through the ring)
       if (fl.remnant) v.rem[f + F * k] = gp;
     }
     cp_prev = cp;
@@ -335,7 +334,7 @@ __global__ void __launch_bounds__(MTPB) k_vdiff_momentum(MomView vu, MomView vv,
     // beyond nz leave every row the identity, and the loops below are empty)
     const int kk = min(max(k, k_lo), nz - 1);
     q.c = v.cd[f + F * kk];
-    if (fl.solve) q.d = v.rd[f + F * kk];
+    if (fl.solve) q.d = v.u[f + F * kk];
     if (fl.remnant) q.g = v.rem[f + F * kk];
   };
   Back br[MPF];
@@ -394,7 +393,6 @@ struct MomState {
   double* tau_v = nullptr;
   long long tau_gen = -1;  // the handle's tau_gen tau_u, tau_v were copied at (-1: never)
   double* cd = nullptr;    // [nz][Fu] then [nz][Fv]
-  double* rd = nullptr;
   double* rem_u = nullptr;
   double* rem_v = nullptr;
   bool rem_valid = false;
@@ -568,7 +566,6 @@ int mom_solve(rdb_colphys* h, double dt, const rdb_colphys_momentum_config* c) {
     if (!st) st = mom_alloc(h, &m->tau_u, 8 * m->Fu);
     if (!st) st = mom_alloc(h, &m->tau_v, 8 * m->Fv);
     if (!st) st = mom_alloc(h, &m->cd, 8 * nz * (m->Fu + m->Fv));
-    if (!st) st = mom_alloc(h, &m->rd, 8 * nz * (m->Fu + m->Fv));
     if (st) return st;
   }
   if (do_remnant && !m->rem_u) {
@@ -643,7 +640,6 @@ int mom_solve(rdb_colphys* h, double dt, const rdb_colphys_momentum_config* c) {
     v.ktop = m->field(xf ? "k_top_u" : "k_top_v");
     v.kbot = m->field(xf ? "k_bot_u" : "k_bot_v");
     v.cd = m->cd + (xf ? 0 : nz * m->Fu);
-    v.rd = m->rd + (xf ? 0 : nz * m->Fu);
     v.rem = xf ? m->rem_u : m->rem_v;
   }
   // the closure's kv with nothing but the wind stress folded in (the

@@ -9,11 +9,14 @@ tile; and a column step after the momentum solve reads the new velocities.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
 from roundabout_amd import synth
 from roundabout_amd.rdb import ColumnPhysics, default_config
+from roundabout_amd.rdb import remap as R
 
 pytestmark = pytest.mark.gpu
 DT = 3600.0
@@ -177,3 +180,25 @@ def test_bottom_and_top_rows_beyond_the_column(orc, nx, ny, nz, remnant_only):
         cp.vdiff_momentum(DT, use_kv_source=0, **{k: (int(x) if isinstance(x, bool) else x) for k, x in kw.items()})
         for name, want in (("u_face_x_layer", u), ("v_face_y_layer", v), ("visc_rem_u", ru), ("visc_rem_v", rv)):
             assert np.array_equal(cp.get_field(name), want), name
+
+
+def test_work_arrays_of_a_solve():
+    """Beside the face velocities and the natural-order copies of h and kv a
+    solve keeps c' of both directions: no more than two face fields."""
+    nx, ny, nz = 256, 256, 128
+    print(f"[case] momentum: device memory of the first solve, {nx}x{ny}x{nz}", flush=True)
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert R._hip().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    with ColumnPhysics(nx, ny, nz, np.ones((nx, ny), order="F")) as cp:
+        cp.set_field("h_layer", np.full((nx, ny, nz), 10.0, order="F"))
+        cp.step(DT, 1)
+        cp.synchronize()
+        before = free()
+        cp.vdiff_momentum(DT, implicit_stress=1)
+        cp.synchronize()
+        field = 8 * nz * (nx + 1) * ny
+        assert before - free() < 6 * field + (32 << 20)
