@@ -749,7 +749,9 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
   int s = 0, s_first_cell = 0;  // the first cell walked, and the one where the targets begin
   double zs_lo = 0.0;
   if (SPLIT && k0 > 0) {
-    bool rising = true;  // the targets' interfaces
+    // (the highest interface: a negative or NaN target does not take back
+    // what one lane would have passed before it)
+    double zn_max = 0.0;
     for (int j0 = 0; j0 < k0; j0 += 8) {
       double h[8];
 #pragma unroll
@@ -758,44 +760,28 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
       for (int u = 0; u < 8; ++u)
         if (j0 + u < k0) {
           zn_hi = zn_hi + h[u];
-          rising = rising && h[u] >= 0.0;
+          zn_max = zn_hi > zn_max ? zn_hi : zn_max;
         }
     }
+    // the first source cell whose top lies above, and the bottom of the one below it
     double z = 0.0, z_below = 0.0;
-    if (rising) {
-      // the first source cell whose top lies above, and the bottom of the one below it
-      bool found = false;
-      for (int j0 = 0; j0 < nz && !found; j0 += 8) {
-        double h[8];
+    bool found = false;
+    for (int j0 = 0; j0 < nz && !found; j0 += 8) {
+      double h[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) h[u] = cols.src_h(min(j0 + u, nz - 1));
+      for (int u = 0; u < 8; ++u) h[u] = cols.src_h(min(j0 + u, nz - 1));
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (!found && j0 + u < nz) {
-            const double top = z + h[u];
-            if (top <= zn_hi) {
-              s_first_cell = j0 + u + 1;
-              z_below = z;
-              z = top;
-            } else {
-              found = true;
-            }
+      for (int u = 0; u < 8; ++u)
+        if (!found && j0 + u < nz) {
+          const double top = z + h[u];
+          if (top <= zn_max) {
+            s_first_cell = j0 + u + 1;
+            z_below = z;
+            z = top;
+          } else {
+            found = true;
           }
-      }
-    } else {
-      // a negative or NaN target below: the cells that one lane would have
-      // passed on its way here
-      double zn = 0.0;
-      for (int j = 0; j <= k0; ++j) {
-        while (s_first_cell < nz) {
-          const double top = z + cols.src_h(s_first_cell);
-          if (!(top <= zn)) break;
-          ++s_first_cell;
-          z_below = z;
-          z = top;
         }
-        if (j < k0) zn = zn + cols.dst_h(j);
-      }
     }
     s = s_first_cell > 0 ? s_first_cell - 1 : 0;
     zs_lo = s_first_cell > 0 ? z_below : 0.0;
