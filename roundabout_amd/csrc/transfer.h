@@ -11,8 +11,10 @@ namespace colphys {
 
 // One engine serves a handle (an ensemble's members share their parent's)
 // and goes with it; one transfer runs at a time.  Four pinned chunks of
-// 4 MiB (16 after a transfer of 64 MiB and more) and up to seven threads,
-// asleep between transfers, are made at the first large transfer.
+// 4 MiB (16 after a transfer of 64 MiB and more) and up to seven threads are
+// made at the first large transfer.  The threads are asleep but for some tens
+// of microseconds after a chunk: the calling thread alone waits for the work
+// that the stream holds.
 //
 // hipMemcpy on pageable memory copies through the runtime's own pinned
 // buffer with the calling thread alone.  That thread's memcpy bounds it, and

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
@@ -36,94 +37,85 @@ int allowed_cpus() {
   return sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
 }
 
-// a short wait for a condition that another running thread is about to set
+// A short wait for a condition that another running thread is about to set:
+// tens of microseconds, then the caller sleeps on a condition variable.
 template <class Cond>
-void spin_until(Cond cond) {
-  for (int i = 0; !cond(); ++i)
-    if (i > 2000) sched_yield();
+bool spin_for(Cond cond) {
+  constexpr auto SPIN = std::chrono::microseconds(50);
+  const auto end = std::chrono::steady_clock::now() + SPIN;
+  for (int i = 0;; ++i) {
+    if (cond()) return true;
+    if (i % 16 == 15 && std::chrono::steady_clock::now() > end) return false;
+  }
 }
 
 }  // namespace
 
 struct Transfer::Impl {
   std::mutex call;  // one transfer at a time
-  // the threads sleep on `cv` between transfers; during one, chunk i is
-  // theirs to copy when `open` > i, and `left[i % NSLOT]` of them still work
-  // on it
+  // The threads copy a block at a time, each its part, and are woken only
+  // when the bytes are there: a wait for the stream (the work queued before
+  // the transfer, which may take seconds) is the calling thread's alone.
   std::mutex m;
-  std::condition_variable cv;
+  std::condition_variable cv, cv_done;
   std::vector<std::thread> threads;
   int n_threads = 0;  // 0: not started
-  uint64_t job = 0;
+  int sleeping = 0;
   bool quit = false;
-  char* dst = nullptr;        // null: the slot
-  const char* src = nullptr;  // null: the slot
+  std::atomic<uint64_t> turn{0};  // bumped for each block
+  std::atomic<int> left{0};       // threads still on it
+  char* dst = nullptr;
+  const char* src = nullptr;
   size_t bytes = 0;
-  std::atomic<size_t> open{0};
-  std::atomic<int> left[NSLOT];
-  std::atomic<int> running{0};
   // pinned chunks, made at the first transfer that needs them
   char* slot[NSLOT] = {nullptr, nullptr, nullptr, nullptr};
   hipEvent_t done[NSLOT] = {nullptr, nullptr, nullptr, nullptr};
   size_t slot_bytes = 0;
-  size_t chunk = SMALL_CHUNK;  // of this transfer
 
   static size_t chunk_of(size_t n) { return n >= BIG ? BIG_CHUNK : SMALL_CHUNK; }
-  size_t chunks() const { return (bytes + chunk - 1) / chunk; }
 
-  // part `t` of `n` of chunk i, in whole pages of 4 KiB where it can be
-  void part(size_t i, int t) {
-    const size_t at = i * chunk, len = std::min(chunk, bytes - at);
-    const size_t per = (len / (size_t)n_threads + 4095) / 4096 * 4096;
-    const size_t a = std::min(len, per * (size_t)t), b = t + 1 == n_threads ? len : std::min(len, per * (size_t)(t + 1));
-    char* const s = slot[i % NSLOT];
-    if (b > a) std::memcpy((dst ? dst + at : s) + a, (src ? src + at : s) + a, b - a);
-    left[i % NSLOT].fetch_sub(1, std::memory_order_release);
+  // part `t` of the block, in whole pages of 4 KiB where it can be
+  void part(int t) {
+    const size_t per = (bytes / (size_t)n_threads + 4095) / 4096 * 4096;
+    const size_t a = std::min(bytes, per * (size_t)t), b = t + 1 == n_threads ? bytes : std::min(bytes, per * (size_t)(t + 1));
+    if (b > a) std::memcpy(dst + a, src + a, b - a);
+    if (left.fetch_sub(1, std::memory_order_acq_rel) == 1) {
+      std::lock_guard<std::mutex> lk(m);
+      cv_done.notify_one();
+    }
   }
 
   void work(int t) {
     uint64_t seen = 0;
     for (;;) {
-      {
+      if (!spin_for([&] { return turn.load(std::memory_order_acquire) != seen; })) {
         std::unique_lock<std::mutex> lk(m);
-        cv.wait(lk, [&] { return quit || job != seen; });
+        ++sleeping;
+        cv.wait(lk, [&] { return quit || turn.load(std::memory_order_acquire) != seen; });
+        --sleeping;
         if (quit) return;
-        seen = job;
       }
-      const size_t n = chunks();
-      for (size_t i = 0; i < n; ++i) {
-        spin_until([&] { return open.load(std::memory_order_acquire) > i; });
-        if (open.load(std::memory_order_acquire) == SIZE_MAX) break;  // the transfer was given up
-        part(i, t);
-      }
-      running.fetch_sub(1, std::memory_order_release);
+      ++seen;  // (the caller waits for every thread before the next turn)
+      part(t);
     }
   }
 
-  void begin(char* d, const char* s, size_t n) {
-    std::lock_guard<std::mutex> lk(m);
-    dst = d;
-    src = s;
+  // A block, copied by the threads and the caller; returns when it is.
+  void share(void* d, const void* s, size_t n) {
+    dst = (char*)d;
+    src = (const char*)s;
     bytes = n;
-    chunk = chunk_of(n);
-    open.store(0, std::memory_order_relaxed);
-    for (auto& l : left) l.store(0, std::memory_order_relaxed);
-    running.store(n_threads - 1, std::memory_order_relaxed);
-    ++job;
-    cv.notify_all();
-  }
-  // hand chunk i out and copy the caller's own part of it
-  void hand_out(size_t i) {
-    left[i % NSLOT].store(n_threads, std::memory_order_relaxed);
-    open.store(i + 1, std::memory_order_release);
-    part(i, 0);
-  }
-  void wait_chunk(size_t i) {
-    spin_until([&] { return left[i % NSLOT].load(std::memory_order_acquire) == 0; });
-  }
-  void end(bool give_up) {
-    if (give_up) open.store(SIZE_MAX, std::memory_order_release);
-    spin_until([&] { return running.load(std::memory_order_acquire) == 0; });
+    left.store(n_threads, std::memory_order_relaxed);
+    turn.fetch_add(1, std::memory_order_release);
+    {
+      std::lock_guard<std::mutex> lk(m);
+      if (sleeping > 0) cv.notify_all();
+    }
+    part(0);
+    if (!spin_for([&] { return left.load(std::memory_order_acquire) == 0; })) {
+      std::unique_lock<std::mutex> lk(m);
+      cv_done.wait(lk, [&] { return left.load(std::memory_order_acquire) == 0; });
+    }
   }
 
   void start() {
@@ -193,17 +185,15 @@ hipError_t Transfer::to_host(void* dst, const void* dev, size_t bytes, hipStream
                                   hipMemcpyDeviceToHost, stream);
     return r == hipSuccess ? hipEventRecord(im.done[i % NSLOT], stream) : r;
   };
-  im.begin((char*)dst, nullptr, bytes);
   size_t sent = 0;
   for (; sent < std::min<size_t>(n, NSLOT) && e == hipSuccess; ++sent) e = fetch(sent);
   for (size_t i = 0; i < n && e == hipSuccess; ++i) {
     e = hipEventSynchronize(im.done[i % NSLOT]);
     if (e != hipSuccess) break;
-    im.hand_out(i);
-    im.wait_chunk(i);
+    const size_t at = i * chunk;
+    im.share((char*)dst + at, im.slot[i % NSLOT], std::min(chunk, bytes - at));
     if (sent < n) e = fetch(sent++);
   }
-  im.end(e != hipSuccess);
   return e;
 }
 
@@ -216,18 +206,15 @@ hipError_t Transfer::to_device(void* dev, const void* src, size_t bytes, hipStre
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
   }
   const size_t chunk = Impl::chunk_of(bytes), n = (bytes + chunk - 1) / chunk;
-  im.begin(nullptr, (const char*)src, bytes);
   for (size_t i = 0; i < n && e == hipSuccess; ++i) {
     // the slot's last transfer, of this call or an earlier one
     e = hipEventSynchronize(im.done[i % NSLOT]);
     if (e != hipSuccess) break;
-    im.hand_out(i);
-    im.wait_chunk(i);
-    const size_t at = i * chunk;
-    e = hipMemcpyAsync((char*)dev + at, im.slot[i % NSLOT], std::min(chunk, bytes - at), hipMemcpyHostToDevice, stream);
+    const size_t at = i * chunk, len = std::min(chunk, bytes - at);
+    im.share(im.slot[i % NSLOT], (const char*)src + at, len);
+    e = hipMemcpyAsync((char*)dev + at, im.slot[i % NSLOT], len, hipMemcpyHostToDevice, stream);
     if (e == hipSuccess) e = hipEventRecord(im.done[i % NSLOT], stream);
   }
-  im.end(e != hipSuccess);
   return e;
 }
 
@@ -239,14 +226,7 @@ void Transfer::copy(void* dst, const void* src, size_t bytes) {
   }
   std::lock_guard<std::mutex> lk(im.call);
   im.start();
-  const size_t chunk = Impl::chunk_of(bytes), n = (bytes + chunk - 1) / chunk;
-  im.begin((char*)dst, (const char*)src, bytes);
-  for (size_t i = 0; i < n; ++i) {
-    if (i >= NSLOT) im.wait_chunk(i - NSLOT);  // its counter is chunk i's
-    im.hand_out(i);
-  }
-  for (size_t i = n > NSLOT ? n - NSLOT : 0; i < n; ++i) im.wait_chunk(i);
-  im.end(false);
+  im.share(dst, src, bytes);
 }
 
 }  // namespace colphys

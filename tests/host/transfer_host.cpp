@@ -1,0 +1,23 @@
+// C entries over colphys::Transfer for tests/test_transfer_host.py.
+#include "../../roundabout_amd/csrc/transfer.h"
+
+extern "C" {
+
+colphys::Transfer* tr_new() { return new colphys::Transfer; }
+void tr_delete(colphys::Transfer* t) { delete t; }
+HostStream* tr_stream() { return new HostStream; }
+void tr_busy(HostStream* s, double seconds) {
+  s->busy_until = std::chrono::steady_clock::now() + std::chrono::microseconds((long long)(1e6 * seconds));
+}
+int tr_to_host(colphys::Transfer* t, void* dst, const void* dev, size_t n, HostStream* s) {
+  return t->to_host(dst, dev, n, s);
+}
+int tr_to_device(colphys::Transfer* t, void* dev, const void* src, size_t n, HostStream* s) {
+  return t->to_device(dev, src, n, s);
+}
+int tr_sync(HostStream* s) { return hipStreamSynchronize(s); }
+void tr_copy(colphys::Transfer* t, void* dst, const void* src, size_t n) { t->copy(dst, src, n); }
+void tr_refuse_pinned(int on) { g_hip.refuse_pinned = on != 0; }
+int tr_last_error() { return hipGetLastError(); }
+
+}  // extern "C"

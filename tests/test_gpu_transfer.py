@@ -6,10 +6,12 @@ and the checks that moved to the device with the upload of h_layer.  Exact."""
 from __future__ import annotations
 
 import ctypes
+import time
 
 import numpy as np
 import pytest
 
+from roundabout_amd import synth
 from roundabout_amd.rdb import ColumnEnsemble, ColumnPhysics, RdbError, _ffi
 from test_gpu_contrib import say
 
@@ -94,3 +96,26 @@ def test_land_contract_is_checked(gpu_lib, nz):
         h[:, :, : nz // 2] = np.minimum(h[:, :, : nz // 2], 1e-4)  # fillers
         cp.set_field("h_layer", h)
         assert cp.stats()["live_levels"] == int((wet > 0.5).sum()) * (nz - nz // 2)
+
+
+@pytest.mark.parametrize("way", ["get", "set"])
+def test_one_thread_waits_for_the_steps_in_flight(gpu_lib, way):
+    """A copy behind steps that are still running costs one thread's wait."""
+    say(f"[case] transfer: {way}_field behind a long run")
+    nx, ny, nz = 480, 360, 75
+    o = synth.make_ocean(nx, ny, nz, 1, land_frac=0.3, topo="zlevel", dmin=50.0, dmax=5500.0)
+    with ColumnPhysics.from_ocean(o) as cp:
+        T = cp.get_field("temperature")
+        for n_steps in (1, 2000):  # once to make the chunks, the threads and the graph
+            cp.set_field("temperature", T)
+            cp.step(3600.0, 1)
+            cp.synchronize()
+            cp.step(3600.0, n_steps)
+            wall, cpu = time.perf_counter(), time.process_time()
+            if way == "get":
+                cp.get_field("temperature")
+            else:
+                cp.set_field("temperature", T)
+            wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    say(f"wall {wall:.3f} s, process CPU {cpu:.3f} s")
+    assert wall > 0.1 and cpu < 2.0 * wall

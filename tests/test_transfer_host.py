@@ -1,0 +1,75 @@
+"""The host side of the copies in pinned chunks (transfer.hip), compiled for
+the CPU against a host stand-in for the HIP calls it makes (tests/host): what
+the copying threads do while the stream is busy."""
+
+from __future__ import annotations
+
+import ctypes
+import subprocess
+import time
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+VP, SZ = ctypes.c_void_p, ctypes.c_size_t
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = tmp_path_factory.mktemp("transfer") / "libtransfer_host.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-pthread", "-I", str(ROOT / "tests/host"), "-x", "c++",
+                    str(ROOT / "roundabout_amd/csrc/transfer.hip"), str(ROOT / "tests/host/transfer_host.cpp"), "-o",
+                    str(so)], check=True)
+    lib = ctypes.CDLL(str(so))
+    lib.tr_new.restype = lib.tr_stream.restype = VP
+    lib.tr_delete.argtypes = lib.tr_sync.argtypes = [VP]
+    lib.tr_busy.argtypes = [VP, ctypes.c_double]
+    lib.tr_to_host.argtypes = lib.tr_to_device.argtypes = [VP, VP, VP, SZ, VP]
+    lib.tr_copy.argtypes = [VP, VP, VP, SZ]
+    return lib
+
+
+@pytest.fixture
+def engine(lib):
+    t = lib.tr_new()
+    yield t
+    lib.tr_delete(t)
+
+
+def _p(a):
+    return a.ctypes.data
+
+
+@pytest.mark.parametrize("n", [1, (1 << 20) - 8, 1 << 20, (1 << 20) + 8, (4 << 20) + 8, (24 << 20) - 3, 64 << 20, (90 << 20) + 5])
+def test_copies_whole(lib, engine, n):
+    rng = np.random.default_rng(n)
+    a = rng.integers(0, 255, n, dtype=np.uint8)
+    dev, out, host = (np.zeros(n, dtype=np.uint8) for _ in range(3))
+    s = lib.tr_stream()
+    for turn in range(3):
+        a ^= 1 + turn
+        assert lib.tr_to_device(engine, _p(dev), _p(a), n, s) == 0
+        assert lib.tr_to_host(engine, _p(out), _p(dev), n, s) == 0
+        lib.tr_copy(engine, _p(host), _p(a), n)
+        assert np.array_equal(out, a) and np.array_equal(host, a)
+
+
+@pytest.mark.parametrize("way", ["to_host", "to_device"])
+def test_threads_sleep_while_the_stream_is_busy(lib, engine, way):
+    """A copy behind a long queue of work costs the time of its memcpys, not
+    every thread's time until the queue has drained."""
+    n = 96 << 20
+    a, dev = np.ones(n, dtype=np.uint8), np.zeros(n, dtype=np.uint8)
+    s = lib.tr_stream()
+    f = lib.tr_to_host if way == "to_host" else lib.tr_to_device
+    for busy in (0.0, 0.6):  # once to make the chunks and the threads
+        lib.tr_sync(s)
+        lib.tr_busy(s, busy)
+        wall, cpu = time.perf_counter(), time.process_time()
+        assert f(engine, _p(a), _p(dev), n, s) == 0
+        wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    lib.tr_sync(s)
+    print(f"{way}: wall {wall:.3f} s, process CPU {cpu:.3f} s")
+    assert wall > 0.5 and cpu < 0.35
