@@ -30,6 +30,7 @@ constexpr size_t SMALL = 1u << 20;
 // 4 MiB, 2.0 of 16 (52 GB/s, the link's rate); down into a fresh array 6.1
 // (10 at worst), 4.6, 2.3 to 3.0.
 constexpr size_t SMALL_CHUNK = 4u << 20, BIG_CHUNK = 16u << 20, BIG = 64u << 20;
+constexpr int PIECES = 32;  // of a block that the threads copy
 
 int allowed_cpus() {
   cpu_set_t set;
@@ -53,20 +54,26 @@ bool spin_for(Cond cond) {
 
 struct Transfer::Impl {
   std::mutex call;  // one transfer at a time
-  // The threads copy a block at a time, each its part, and are woken only
-  // when the bytes are there: a wait for the stream (the work queued before
-  // the transfer, which may take seconds) is the calling thread's alone.
+  // The threads copy a block at a time and are woken only when the bytes are
+  // there: a wait for the stream (the work queued before the transfer, which
+  // may take seconds) is the calling thread's alone.  A block is cut into
+  // 32 pieces; each thread has a run of its own, the same one in every block
+  // (its processor's caches and a huge page of a fresh destination), and goes
+  // on to what others have not begun, so that one that is late or loses its
+  // processor holds up no more than the piece it is at.
   std::mutex m;
   std::condition_variable cv, cv_done;
   std::vector<std::thread> threads;
+  bool quit = false, caller_waits = false;
   int n_threads = 0;  // 0: not started
   int sleeping = 0;
-  bool quit = false;
-  std::atomic<uint64_t> turn{0};  // bumped for each block
-  std::atomic<int> left{0};       // threads still on it
+  // the block's number in the high half, a bit for each piece not yet taken in
+  // the low one: nothing is taken of a block that is done, whatever came after
+  std::atomic<uint64_t> open{0};
+  std::atomic<int> left{0};  // pieces not yet copied; at 0 the next block may be set up
   char* dst = nullptr;
   const char* src = nullptr;
-  size_t bytes = 0;
+  size_t bytes = 0, piece = 0;
   // pinned chunks, made at the first transfer that needs them
   char* slot[NSLOT] = {nullptr, nullptr, nullptr, nullptr};
   hipEvent_t done[NSLOT] = {nullptr, nullptr, nullptr, nullptr};
@@ -74,29 +81,41 @@ struct Transfer::Impl {
 
   static size_t chunk_of(size_t n) { return n >= BIG ? BIG_CHUNK : SMALL_CHUNK; }
 
-  // part `t` of the block, in whole pages of 4 KiB where it can be
-  void part(int t) {
-    const size_t per = (bytes / (size_t)n_threads + 4095) / 4096 * 4096;
-    const size_t a = std::min(bytes, per * (size_t)t), b = t + 1 == n_threads ? bytes : std::min(bytes, per * (size_t)(t + 1));
-    if (b > a) std::memcpy(dst + a, src + a, b - a);
+  // the pieces that are thread t's own (the caller is thread 0 of n)
+  static uint32_t own_of(int t, int n) {
+    const int a = PIECES * t / n, b = PIECES * (t + 1) / n;
+    return (uint32_t)((1ull << b) - (1ull << a));
+  }
+  // take a piece, of `own` before others', and copy it; false if there is none
+  bool take(uint32_t own) {
+    uint64_t o = open.load(std::memory_order_acquire);
+    int k;
+    do {
+      const uint32_t mine = (uint32_t)o & own;
+      if ((uint32_t)o == 0) return false;
+      k = mine ? __builtin_ctz(mine) : 31 - __builtin_clz((uint32_t)o);
+    } while (!open.compare_exchange_weak(o, o & ~(1ull << k), std::memory_order_acq_rel, std::memory_order_acquire));
+    const size_t at = piece * (size_t)k;
+    std::memcpy(dst + at, src + at, std::min(piece, bytes - at));
     if (left.fetch_sub(1, std::memory_order_acq_rel) == 1) {
       std::lock_guard<std::mutex> lk(m);
-      cv_done.notify_one();
+      if (caller_waits) cv_done.notify_one();
     }
+    return true;
   }
+  bool some() const { return (uint32_t)open.load(std::memory_order_acquire) != 0; }
 
-  void work(int t) {
-    uint64_t seen = 0;
+  void work(int t, int n) {
+    const uint32_t own = own_of(t, n);
     for (;;) {
-      if (!spin_for([&] { return turn.load(std::memory_order_acquire) != seen; })) {
-        std::unique_lock<std::mutex> lk(m);
-        ++sleeping;
-        cv.wait(lk, [&] { return quit || turn.load(std::memory_order_acquire) != seen; });
-        --sleeping;
-        if (quit) return;
+      while (take(own)) {
       }
-      ++seen;  // (the caller waits for every thread before the next turn)
-      part(t);
+      if (spin_for([&] { return some(); })) continue;
+      std::unique_lock<std::mutex> lk(m);
+      ++sleeping;
+      cv.wait(lk, [&] { return quit || some(); });
+      --sleeping;
+      if (quit) return;
     }
   }
 
@@ -105,16 +124,23 @@ struct Transfer::Impl {
     dst = (char*)d;
     src = (const char*)s;
     bytes = n;
-    left.store(n_threads, std::memory_order_relaxed);
-    turn.fetch_add(1, std::memory_order_release);
+    piece = (n / PIECES + 4096) / 4096 * 4096;
+    const int pieces = (int)((n + piece - 1) / piece);
+    left.store(pieces, std::memory_order_relaxed);
+    const uint64_t number = (open.load(std::memory_order_relaxed) >> 32) + 1;
+    open.store(number << 32 | ((1ull << pieces) - 1), std::memory_order_release);
     {
       std::lock_guard<std::mutex> lk(m);
       if (sleeping > 0) cv.notify_all();
     }
-    part(0);
+    const uint32_t own = own_of(0, n_threads);
+    while (take(own)) {
+    }
     if (!spin_for([&] { return left.load(std::memory_order_acquire) == 0; })) {
       std::unique_lock<std::mutex> lk(m);
+      caller_waits = true;
       cv_done.wait(lk, [&] { return left.load(std::memory_order_acquire) == 0; });
+      caller_waits = false;
     }
   }
 
@@ -122,11 +148,11 @@ struct Transfer::Impl {
     if (n_threads > 0) return;
     const int want = std::max(1, std::min(MAX_THREADS, allowed_cpus() / 2));
     try {
-      for (int t = 1; t < want; ++t) threads.emplace_back([this, t] { work(t); });
+      for (int t = 1; t < want; ++t) threads.emplace_back([this, t, want] { work(t, want); });
     } catch (const std::system_error&) {
       // fewer threads than wanted: those there are do the work
     }
-    n_threads = (int)threads.size() + 1;
+    n_threads = want;  // (the shares of threads that are not there are taken by the others)
   }
   hipError_t prepare(size_t n) {
     start();
@@ -226,7 +252,8 @@ void Transfer::copy(void* dst, const void* src, size_t bytes) {
   }
   std::lock_guard<std::mutex> lk(im.call);
   im.start();
-  im.share(dst, src, bytes);
+  for (size_t at = 0; at < bytes; at += BIG)
+    im.share((char*)dst + at, (const char*)src + at, std::min(BIG, bytes - at));
 }
 
 }  // namespace colphys

@@ -1,6 +1,18 @@
 // C entries over colphys::Transfer for tests/test_transfer_host.py.
 #include "../../roundabout_amd/csrc/transfer.h"
 
+#include <signal.h>
+#include <sys/syscall.h>
+#include <time.h>
+#include <unistd.h>
+
+static int hold_ms = 0;
+static void hold(int) {
+  timespec t{hold_ms / 1000, (hold_ms % 1000) * 1000000L};
+  while (nanosleep(&t, &t) != 0) {
+  }
+}
+
 extern "C" {
 
 colphys::Transfer* tr_new() { return new colphys::Transfer; }
@@ -17,6 +29,12 @@ int tr_to_device(colphys::Transfer* t, void* dev, const void* src, size_t n, Hos
 }
 int tr_sync(HostStream* s) { return hipStreamSynchronize(s); }
 void tr_copy(colphys::Transfer* t, void* dst, const void* src, size_t n) { t->copy(dst, src, n); }
+// thread `tid` of this process stands still for `ms`
+void tr_hold(int tid, int ms) {
+  hold_ms = ms;
+  signal(SIGUSR2, hold);
+  syscall(SYS_tgkill, getpid(), tid, SIGUSR2);
+}
 void tr_refuse_pinned(int on) { g_hip.refuse_pinned = on != 0; }
 int tr_last_error() { return hipGetLastError(); }
 

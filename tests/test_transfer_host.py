@@ -5,6 +5,7 @@ the copying threads do while the stream is busy."""
 from __future__ import annotations
 
 import ctypes
+import os
 import subprocess
 import time
 from pathlib import Path
@@ -73,3 +74,24 @@ def test_threads_sleep_while_the_stream_is_busy(lib, engine, way):
     lib.tr_sync(s)
     print(f"{way}: wall {wall:.3f} s, process CPU {cpu:.3f} s")
     assert wall > 0.5 and cpu < 0.35
+
+
+def test_a_thread_that_is_held_up_holds_up_nothing(lib, engine):
+    """One of the copying threads loses its processor (a signal handler that
+    sleeps): the others do its share."""
+    n = 32 << 20
+    a, b = np.arange(n, dtype=np.uint8), np.zeros(n, dtype=np.uint8)
+    before = set(os.listdir("/proc/self/task"))
+    lib.tr_copy(engine, _p(b), _p(a), n)
+    helpers = sorted(set(os.listdir("/proc/self/task")) - before)
+    assert helpers, "no copying thread (one processor?)"
+    time.sleep(0.02)
+    b[...] = 0
+    lib.tr_hold(int(helpers[0]), 800)
+    time.sleep(0.02)
+    wall = time.perf_counter()
+    lib.tr_copy(engine, _p(b), _p(a), n)
+    wall = time.perf_counter() - wall
+    print(f"wall {wall:.3f} s with one of {len(helpers)} threads held for 0.8 s")
+    assert np.array_equal(a, b) and wall < 0.4
+    time.sleep(0.9)  # the handler returns before the engine goes
