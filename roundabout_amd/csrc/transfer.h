@@ -13,8 +13,8 @@ namespace colphys {
 // and goes with it; one transfer runs at a time.  Four pinned chunks of
 // 4 MiB (16 after a transfer of 64 MiB and more) and up to seven threads are
 // made at the first large transfer.  The threads are asleep but for some tens
-// of microseconds after a chunk: the calling thread alone waits for the work
-// that the stream holds.
+// of microseconds at the start of a transfer and after a chunk: the calling
+// thread alone waits for the work that the stream holds.
 //
 // hipMemcpy on pageable memory copies through the runtime's own pinned
 // buffer with the calling thread alone.  That thread's memcpy bounds it, and

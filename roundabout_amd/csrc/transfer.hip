@@ -31,6 +31,7 @@ constexpr size_t SMALL = 1u << 20;
 // (10 at worst), 4.6, 2.3 to 3.0.
 constexpr size_t SMALL_CHUNK = 4u << 20, BIG_CHUNK = 16u << 20, BIG = 64u << 20;
 constexpr int PIECES = 32;  // of a block that the threads copy
+constexpr size_t WORTH = 512u << 10;  // bytes for which one more thread is woken
 
 int allowed_cpus() {
   cpu_set_t set;
@@ -67,6 +68,7 @@ struct Transfer::Impl {
   bool quit = false, caller_waits = false;
   int n_threads = 0;  // 0: not started
   int sleeping = 0;
+  uint64_t calls = 0;  // bumped by call_up
   // the block's number in the high half, a bit for each piece not yet taken in
   // the low one: nothing is taken of a block that is done, whatever came after
   std::atomic<uint64_t> open{0};
@@ -107,17 +109,36 @@ struct Transfer::Impl {
 
   void work(int t, int n) {
     const uint32_t own = own_of(t, n);
+    uint64_t heard = 0;
     for (;;) {
       while (take(own)) {
       }
       if (spin_for([&] { return some(); })) continue;
       std::unique_lock<std::mutex> lk(m);
       ++sleeping;
-      cv.wait(lk, [&] { return quit || some(); });
+      cv.wait(lk, [&] { return quit || some() || calls != heard; });
       --sleeping;
+      heard = calls;
       if (quit) return;
     }
   }
+
+  // Wake as many threads as `n` bytes are worth: a wake-up costs the thread
+  // some tens of microseconds, and the caller some of its own for each call.
+  void wake(size_t n, bool ahead = false) {
+    std::lock_guard<std::mutex> lk(m);
+    if (ahead) ++calls;
+    if (sleeping == 0) return;
+    const size_t want = n / WORTH;
+    if (2 * want >= (size_t)sleeping)
+      cv.notify_all();
+    else
+      for (size_t i = 0; i < want; ++i) cv.notify_one();
+  }
+
+  // A chunk of `n` bytes may be here soon: the threads' way out of their sleep
+  // overlaps its transfer.  (If it is not, they are back asleep in 50 us.)
+  void call_up(size_t n) { wake(n, true); }
 
   // A block, copied by the threads and the caller; returns when it is.
   void share(void* d, const void* s, size_t n) {
@@ -129,10 +150,7 @@ struct Transfer::Impl {
     left.store(pieces, std::memory_order_relaxed);
     const uint64_t number = (open.load(std::memory_order_relaxed) >> 32) + 1;
     open.store(number << 32 | ((1ull << pieces) - 1), std::memory_order_release);
-    {
-      std::lock_guard<std::mutex> lk(m);
-      if (sleeping > 0) cv.notify_all();
-    }
+    wake(n);
     const uint32_t own = own_of(0, n_threads);
     while (take(own)) {
     }
@@ -213,6 +231,7 @@ hipError_t Transfer::to_host(void* dst, const void* dev, size_t bytes, hipStream
   };
   size_t sent = 0;
   for (; sent < std::min<size_t>(n, NSLOT) && e == hipSuccess; ++sent) e = fetch(sent);
+  im.call_up(std::min(chunk, bytes));
   for (size_t i = 0; i < n && e == hipSuccess; ++i) {
     e = hipEventSynchronize(im.done[i % NSLOT]);
     if (e != hipSuccess) break;
