@@ -194,6 +194,16 @@ struct Transfer::Impl {
     slot_bytes = need;
     return hipSuccess;
   }
+  // Whether a transfer of `n` bytes goes through the chunks.  Where they are
+  // not to be had it does not, and that is no error: what the failed call
+  // left for hipGetLastError goes with it, or the next launch's check would
+  // find it.
+  bool takes(size_t n) {
+    if (n < SMALL) return false;
+    if (prepare(n) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
 };
 
 Transfer::Transfer() : im_(new Impl) {}
@@ -217,8 +227,8 @@ Transfer::~Transfer() {
 hipError_t Transfer::to_host(void* dst, const void* dev, size_t bytes, hipStream_t stream) {
   Impl& im = *im_;
   std::lock_guard<std::mutex> lk(im.call);
-  hipError_t e = bytes < SMALL ? hipSuccess : im.prepare(bytes);
-  if (bytes < SMALL || e != hipSuccess) {
+  hipError_t e = hipSuccess;
+  if (!im.takes(bytes)) {
     e = hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, stream);
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
   }
@@ -245,8 +255,8 @@ hipError_t Transfer::to_host(void* dst, const void* dev, size_t bytes, hipStream
 hipError_t Transfer::to_device(void* dev, const void* src, size_t bytes, hipStream_t stream) {
   Impl& im = *im_;
   std::lock_guard<std::mutex> lk(im.call);
-  hipError_t e = bytes < SMALL ? hipSuccess : im.prepare(bytes);
-  if (bytes < SMALL || e != hipSuccess) {
+  hipError_t e = hipSuccess;
+  if (!im.takes(bytes)) {
     e = hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, stream);
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
   }

@@ -95,3 +95,21 @@ def test_a_thread_that_is_held_up_holds_up_nothing(lib, engine):
     print(f"wall {wall:.3f} s with one of {len(helpers)} threads held for 0.8 s")
     assert np.array_equal(a, b) and wall < 0.4
     time.sleep(0.9)  # the handler returns before the engine goes
+
+
+def test_without_pinned_memory_no_error_is_left(lib):
+    """No pinned chunks to be had: the runtime's own copy is taken, and the
+    failed allocation is not left for the next hipGetLastError to report."""
+    n = 5 << 20
+    a, dev, out = np.full(n, 7, dtype=np.uint8), np.zeros(n, dtype=np.uint8), np.zeros(n, dtype=np.uint8)
+    t, s = lib.tr_new(), lib.tr_stream()
+    lib.tr_refuse_pinned(1)
+    try:
+        assert lib.tr_to_device(t, _p(dev), _p(a), n, s) == 0 and lib.tr_last_error() == 0
+        assert lib.tr_to_host(t, _p(out), _p(dev), n, s) == 0 and lib.tr_last_error() == 0
+    finally:
+        lib.tr_refuse_pinned(0)
+    assert np.array_equal(out, a)
+    out[...] = 0
+    assert lib.tr_to_host(t, _p(out), _p(dev), n, s) == 0 and np.array_equal(out, a)  # there is some again
+    lib.tr_delete(t)
