@@ -9,8 +9,8 @@
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -167,8 +167,8 @@ struct Transfer::Impl {
     const int want = std::max(1, std::min(MAX_THREADS, allowed_cpus() / 2));
     try {
       for (int t = 1; t < want; ++t) threads.emplace_back([this, t, want] { work(t, want); });
-    } catch (const std::system_error&) {
-      // fewer threads than wanted: those there are do the work
+    } catch (const std::exception&) {
+      // no thread or no memory for one, and the callers are C: fewer threads than wanted: those there are do the work
     }
     n_threads = want;  // (the shares of threads that are not there are taken by the others)
   }

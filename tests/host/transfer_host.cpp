@@ -1,10 +1,22 @@
 // C entries over colphys::Transfer for tests/test_transfer_host.py.
 #include "../../roundabout_amd/csrc/transfer.h"
 
+#include <new>
+
 #include <signal.h>
 #include <sys/syscall.h>
 #include <time.h>
 #include <unistd.h>
+
+// operator new of this library alone (linked -Bsymbolic)
+static bool no_memory = false;
+void* operator new(size_t n) {
+  void* const p = no_memory ? nullptr : std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 static int hold_ms = 0;
 static void hold(int) {
@@ -35,6 +47,7 @@ void tr_hold(int tid, int ms) {
   signal(SIGUSR2, hold);
   syscall(SYS_tgkill, getpid(), tid, SIGUSR2);
 }
+void tr_no_memory(int on) { no_memory = on != 0; }
 void tr_refuse_pinned(int on) { g_hip.refuse_pinned = on != 0; }
 int tr_last_error() { return hipGetLastError(); }
 

@@ -20,7 +20,7 @@ VP, SZ = ctypes.c_void_p, ctypes.c_size_t
 @pytest.fixture(scope="module")
 def lib(tmp_path_factory):
     so = tmp_path_factory.mktemp("transfer") / "libtransfer_host.so"
-    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-pthread", "-I", str(ROOT / "tests/host"), "-x", "c++",
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-pthread", "-Wl,-Bsymbolic", "-I", str(ROOT / "tests/host"), "-x", "c++",
                     str(ROOT / "roundabout_amd/csrc/transfer.hip"), str(ROOT / "tests/host/transfer_host.cpp"), "-o",
                     str(so)], check=True)
     lib = ctypes.CDLL(str(so))
@@ -112,4 +112,15 @@ def test_without_pinned_memory_no_error_is_left(lib):
     assert np.array_equal(out, a)
     out[...] = 0
     assert lib.tr_to_host(t, _p(out), _p(dev), n, s) == 0 and np.array_equal(out, a)  # there is some again
+    lib.tr_delete(t)
+
+
+def test_without_memory_for_threads_the_caller_copies(lib):
+    n = 5 << 20
+    a, out = np.full(n, 3, dtype=np.uint8), np.zeros(n, dtype=np.uint8)
+    t = lib.tr_new()
+    lib.tr_no_memory(1)
+    lib.tr_copy(t, _p(out), _p(a), n)  # std::bad_alloc through the C entry would end the process
+    lib.tr_no_memory(0)
+    assert np.array_equal(out, a)
     lib.tr_delete(t)
