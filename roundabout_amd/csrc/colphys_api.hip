@@ -22,6 +22,7 @@
 
 #include "../../include/rdb_colphys.h"
 #include "colphys_handle.h"
+#include "launch_shape.h"
 #include "colphys_kernels.h"
 
 using colphys::Params;
@@ -1488,18 +1489,12 @@ int rdb_colphys_autotune(rdb_colphys* h, double dt) {
       }
     }
   };
-  // candidates: launch block x live levels of Thomas state held in LDS
-  // (up to the device's LDS per workgroup) x column packing (single grids: the
-  // current order, grid order, and deepest-first by live levels, which
-  // keeps a wavefront's columns of one depth together)
+  // candidates: the current shape and others (launch block x live levels of
+  // Thomas state held in LDS, up to the device's LDS per workgroup) x column
+  // packing (single grids: the current order, grid order, and deepest-first
+  // by live levels, which keeps a wavefront's columns of one depth together)
   const size_t nq = (size_t)(3 + std::min(h->n_passive, 4) + (h->cfg.kt_bg != h->cfg.ks_bg ? 1 : 0));
-  std::vector<std::pair<int, int>> cands;
-  for (int b : {64, 128, 256}) {
-    int mmax = (int)((size_t)h->lds_max / ((size_t)b * nq * 8));
-    for (int m : {0, 4, 8, 12, 16, 24, 32}) {
-      if (m <= mmax) cands.push_back({b, m});
-    }
-  }
+  const std::vector<std::pair<int, int>> cands = colphys::shape_candidates(h->lds_max, nq, h->block, h->lds_levels);
   std::vector<std::vector<int>> orders{std::vector<int>(h->col_host.begin(), h->col_host.begin() + h->n_wet)};
   std::vector<int> order_modes{h->order_mode};
   if (h->members.empty() && h->col_live.size() == (size_t)h->n_all) {
