@@ -6,7 +6,8 @@ Grids from one column to a few workgroups, one to six live layers over up to
 88 fillers, mixing depths below and above the column's; the small grids leave
 the foreseen sweeps fewer scratch columns than they have guesses, so the
 sequential sweeps run as well.  Each handle solves four times: the list of
-such columns has to be empty again after every solve.
+such columns has to be empty again after every solve.  One grid lists more
+columns than the launch's workgroups take in one turn.
 """
 
 from __future__ import annotations
@@ -60,3 +61,21 @@ def test_bed_limited_columns(orc, gpu_lib, nx, ny, nz, live_max, knobs):
             ref.step(DT, 1)
             _compare(cp, ref, cfg)
     _assert_equal("wet columns keep their thickness", o.h, ref.ocean.h)
+
+
+def test_more_columns_than_one_turn(orc, gpu_lib):
+    """256 workgroups of 64 columns: a list of more than 16 384 columns makes
+    them go round again, over the same shared arrays and further scratch.  A
+    column of one layer over 13 fillers is listed before its first interface."""
+    nx, ny, nz = 210, 150, 14
+    say(f"[case] EPBL over fillers {nx}x{ny}x{nz}, more than 16384 columns")
+    cfg = default_config()
+    cfg.epbl_enable = 1
+    o = _shallow(nx, ny, nz, 6, 1)
+    assert (o.wet > 0.5).sum() > 16384 + 64
+    ref = orc.OracleState(o, cfg)
+    with ColumnPhysics.from_ocean(o, config=cfg) as cp:
+        for _ in range(2):
+            cp.step(DT, 1)
+            ref.step(DT, 1)
+            _compare(cp, ref, cfg)
