@@ -651,20 +651,21 @@ __global__ __launch_bounds__(TPB) void k_pqm_coeffs(Cols cols, long ncol, int nz
 // ocean_remap_tracer_field (donor column, filler excess, bounding, budget);
 // otherwise the plain remap_column of the face and raw-column passes.
 //
-// What bounds it is issue: on 1440 x 1080 x 75 (PPM, tracers and faces) 508
-// vector instructions a level and wavefront before the kept quotient and the
-// shared way on to the next cell, 442 now, the vector pipes busy two thirds of
-// the time; 2.50 -> 2.26 ms a tracer, and 0.35 ms of copy-back gone in place.
-// (Levels in blocks through LDS, one round trip for four of them, cost more
-// instructions than the latency they hid: 2.6 ms.)
+// What bounds it is issue.  Each overlap divides anew where it begins in its
+// cell: the quotient kept from where the last target ended (a register pair
+// and a flag) cost more than it saved, 440 us against 328 for PLM of
+// 400 000 x 75 columns, and would not hold after a target of negative
+// thickness.  (Levels in blocks through LDS, one round trip for four of them,
+// cost more instructions than the latency they hid.)
 //
-// In place (scratch given: cols' field is out itself) target k may be
+// IN_PLACE (cols' field is out itself; scratch given) target k may be
 // written once level k has gone through the window (k <= s + 2): everything
 // read later lies above.  A lane whose targets run ahead of its sources
 // further than that writes to scratch from there on and copies those levels
-// at its end.  The excesses of a target with more than two filler
-// contributors, which are otherwise gathered from the field again, go to
-// scratch as well, from level 0 up: the j-th of them comes with a source cell
+// at its end, eight at a time (one by one 20 us of 189 on 100 000 x 75, PLM,
+// targets 20 % off their sources).  The excesses of a target with more than
+// two filler contributors, which are otherwise gathered from the field again,
+// go to scratch as well, from level 0 up: the j-th of them comes with a source cell
 // s >= j, so a deferred target that it displaces has its level behind the
 // window and is written out first.  One field of scratch serves both.
 //
@@ -672,8 +673,9 @@ __global__ __launch_bounds__(TPB) void k_pqm_coeffs(Cols cols, long ncol, int nz
 // column, each with a run of the targets: such a lane adds up the thicknesses below
 // (the same running sums) to where its targets begin, and starts the walk one
 // source cell early for the edge that the first one takes over.  Not in
-// place: other lanes' targets are this one's sources.
-template <class Cols, int M, bool FIELD, bool SPLIT>
+// place: other lanes' targets are this one's sources.  (Each way of its own,
+// at compile time: the tests of scratch cost an out-of-place walk 3 to 5 %.)
+template <class Cols, int M, bool FIELD, bool SPLIT, bool IN_PLACE>
 __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, int be, int nu,
                                               const double* __restrict__ W, long arr, double* out,
                                               double* __restrict__ budget, double* __restrict__ clamp,
@@ -797,11 +799,6 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
   // reconstruction of cell s: PLM slope in ra; PPM/H4 (q_L, q_R, q6) in
   // (ra, rb, r6); PQM coefficients in (ra, rb, r6, rd, re)
   double ra = 0.0, rb = 0.0, r6 = 0.0, rd = 0.0, re = 0.0, carry = 0.0;
-  // the position in cell s where the last overlap with it ended, and the
-  // next begins: the quotient of the same operands, kept (not across a target
-  // of no or negative thickness, which may move the next one's bottom back)
-  double x_end = 0.0;
-  bool x_kept = false;
 
   auto recon = [&]() {
     if (M == M_PLM) {
@@ -904,7 +901,6 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
     pb = raw(s + 4);
     zs_lo = zs_hi;
     zs_hi = zs_lo + w1.h;
-    x_kept = false;
     if (s < nz) recon();
   };
   recon();
@@ -921,7 +917,6 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
     const double b_old = (FIELD && budget) ? budget[at] : 0.0;
     const double zn_lo = zn_hi;
     zn_hi = zn_lo + hn;
-    if (!(hn > 0.0)) x_kept = false;
     // the first source cell whose top lies above the target's bottom
     while (s < nz && zs_hi <= zn_lo) advance();
     const double fallback = (s < nz) ? w1.co : w0.co;  // c_own(min(ko0, nz))
@@ -943,10 +938,8 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
           // bottom 0 / h = 0
           double xl = 0.0, xh = 0.0;
           if (M != M_PCM) {
-            if (z_lo != zs_lo) xl = x_kept ? x_end : (z_lo - zs_lo) / w1.h;
+            if (z_lo != zs_lo) xl = (z_lo - zs_lo) / w1.h;
             xh = (z_hi - zs_lo) / w1.h;
-            x_end = xh;
-            x_kept = true;
           }
           if (M == M_PCM) {
             integral = integral + w1.cd * ov;
@@ -985,7 +978,7 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
                   ex0 = sx * ov;
                 else if (n_ex == 1)
                   ex1 = sx * ov;
-                else if (scratch) {
+                else if (IN_PLACE) {
                   const int j = n_ex - 2;
                   const long to = col + ncol * (long)j;
                   if (j >= defer && j < k) {  // (j == defer: the ones below went first)
@@ -1021,15 +1014,15 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
     else
       q = (hn > 0.0) ? integral / hn : 0.0;
     // in place: is level k still to be read?
-    if (scratch && defer == nz && k > s + 2) defer = k;
-    double* const to = (scratch && k >= defer) ? scratch : out;
+    if (IN_PLACE && defer == nz && k > s + 2) defer = k;
+    double* const to = (IN_PLACE && k >= defer) ? scratch : out;
     if (!FIELD) {
       __builtin_nontemporal_store(q, &to[at]);
       continue;
     }
     // remap_add_filler_excess: each filler contributor's own excess, after
     // the division, in source order
-    if (n_ex <= 2 || scratch) {
+    if (n_ex <= 2 || IN_PLACE) {
       if (n_ex > 0) q = q + ex0 / hn;
       if (n_ex > 1) q = q + ex1 / hn;
       for (int j = 2; j < n_ex; ++j) q = q + scratch[col + ncol * (long)(j - 2)] / hn;
@@ -1081,10 +1074,14 @@ __global__ __launch_bounds__(TPB, 4) void k_walk(Cols cols, long ncol, int nz, i
     }
     __builtin_nontemporal_store(cn, &to[at]);  // after the read of its own source cell
   }
-  if (scratch)
-    for (int k = defer; k < nz; ++k) {
-      const long at = col + ncol * (long)k;
-      out[at] = scratch[at];
+  if (IN_PLACE)
+    for (int j0 = defer; j0 < nz; j0 += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = scratch[col + ncol * (long)min(j0 + u, nz - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (j0 + u < nz) out[col + ncol * (long)(j0 + u)] = v[u];
     }
 }
 
@@ -1252,7 +1249,13 @@ int effective_method(int method, int nz) {
 
 // Lanes a column of the walk: one where the columns alone put two wavefronts
 // on every SIMD (256 CUs of four; 131 072 columns), else as many as do, of at
-// least four targets each (1000 columns x 33, PPM_H4: 80 us, 20 split).
+// least four targets each.  us of a column batch, one lane -> split, out of
+// place (in place, where the split walk goes through a buffer):
+//                        20 levels, PLM           33, PPM_H4          75, PLM
+//    1 000 columns   31 -> 11 (32 -> 14)   87 -> 21 (88 -> 23)   120 -> 19 (136 -> 22)
+//   16 000           31 -> 13 (32 -> 19)   88 -> 31 (91 -> 36)   139 -> 41 (165 -> 48)
+//   44 000           32 -> 23 (33 -> 31)   95 -> 73 (99 -> 82)   153 -> 95 (179 -> 106)
+//   65 536           34 -> 25 (34 -> 33)   94 -> 73 (101 -> 82)  159 -> 98 (186 -> 113)
 int walk_splits(long ncol, int nz) {
   const long want = 131072 / ncol;
   return (int)(want < 1 ? 1 : want > nz / 4 ? (nz / 4 > 1 ? nz / 4 : 1) : want);
@@ -1283,11 +1286,13 @@ int launch(const Cols& cols, long ncol, int nz, int method, int be, int nu, doub
     hipLaunchKernelGGL((k_pqm_coeffs<Cols, FIELD>), dim3(grid), dim3(TPB), 0, st, cols, ncol, nz, be, W, arr);
   }
   switch (m) {
-#define RDB_REMAP_CASE(MM)                                                                                        \
+#define RDB_REMAP_CASE(MM)                                                                                      \
   case MM:                                                                                                        \
-    hipLaunchKernelGGL((splits > 1 ? k_walk<Cols, MM, FIELD, true> : k_walk<Cols, MM, FIELD, false>), \
-                       dim3(wgrid, splits), dim3(wtpb), 0, st, cols, ncol, nz, be, nu, W, arr, out, \
-                       budget, clamp, scratch);                                                                            \
+    hipLaunchKernelGGL((splits > 1 ? k_walk<Cols, MM, FIELD, true, false>                                         \
+                        : scratch  ? k_walk<Cols, MM, FIELD, false, true>                                         \
+                                   : k_walk<Cols, MM, FIELD, false, false>),                                      \
+                       dim3(wgrid, splits), dim3(wtpb), 0, st, cols, ncol, nz, be, nu, W, arr, out, budget, clamp, \
+                       scratch);                                                                                  \
     break;
     RDB_REMAP_CASE(M_PCM)
     RDB_REMAP_CASE(M_PLM)
