@@ -16,8 +16,12 @@ namespace colphys {
 // Levels of loads the fused step keeps in flight ahead of its serial
 // sweeps (register ring depth).
 constexpr int PF = 6;
-// The staged tracer solve's.
-constexpr int SPF = 6;
+// The staged tracer solve's: its four right-hand sides fill the registers that
+// a deeper ring would need, and a wavefront more of a SIMD hides as much.  us
+// a solve with 0 (a level loaded when the one before is done), 2, 3 and 6
+// levels: 4096 columns x 20 (T, S) 35, 24, 26, 29; 480 x 360 x 75 (T, S, two
+// passives) 400, 230, 224, 260; 1440 x 1080 x 75 1421, 1297, 1338, 1475.
+constexpr int SPF = 2;
 // Sweep A usually stops a few levels below the surface: a shallower ring.
 constexpr int PFA = 3;
 // Cache policy of the fused step: the streamed inputs of sweep B and the
@@ -359,7 +363,6 @@ __device__ __forceinline__ void solve_group(const StateView& s, const double* __
   // sweeps do (slot j: level kb + j + SPF n going up, nz - 2 - j - SPF n
   // going down; past an end the last level again, unused): a lane that loads
   // level k + 1 when it is done with level k waits a round trip a level.
-  // 480 x 360 x 75, T and S and two passives: 395 -> 270 us.
   struct Up {
     double h, K, x[G];
   };
