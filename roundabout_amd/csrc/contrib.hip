@@ -765,7 +765,10 @@ INST(true)
 // the floors/ceilings of vmix_assemble (rdb_ocean_vmix.F90:2265-2385).  Each
 // is a per-interface update applied in the reference's order, so one pass
 // gives the bits of the separate sweeps; kv, kt and ks are written once.
-constexpr int TAIL = 4;
+// TAIL interfaces' loads are in flight together.  us with 1, 2 and 4 of them:
+// 4096 columns x 20 23, 18, 17; 330 x 300 x 75 257, 197, 191; 480 x 360 x 75
+// 280, 220, 222; 800 x 640 x 60 481, 474, 486; 1440 x 1080 x 75 1710, 1715, 1749.
+constexpr int TAIL = 2;
 __global__ void __launch_bounds__(256) k_coeff_tail(StateView s, Params pr, ContribParams c, EpblView e, int do_pp81, int p0, int p1,
                              unsigned int* guard_count) {
   const int p = p0 + blockIdx.x * blockDim.x + threadIdx.x;
@@ -802,8 +805,7 @@ __global__ void __launch_bounds__(256) k_coeff_tail(StateView s, Params pr, Cont
   double h_up = LV(s.h, nz - 1), rho_up = LV(s.rho, nz - 1);
   double ub_up = do_pp81 ? LV(s.ub, nz - 1) : 0.0, vb_up = do_pp81 ? LV(s.vb, nz - 1) : 0.0;
   double T_up = LV(s.T, nz - 1), S_up = LV(s.S, nz - 1);
-  // the layers below TAIL interfaces at a time, in flight together (one
-  // interface a round trip before: 284 -> 221 us on 480 x 360 x 75)
+  // the layers below TAIL interfaces at a time
   for (int k0 = nz - 1; k0 >= 1; k0 -= TAIL) {
     double bh[TAIL], br[TAIL], bT[TAIL], bS[TAIL], bu[TAIL], bv[TAIL], bk[TAIL];
 #pragma unroll
