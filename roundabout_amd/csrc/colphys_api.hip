@@ -712,8 +712,11 @@ int scan_h(rdb_colphys* h, const double* data) {
 // with nothing in LDS -> this rule: 3 624 columns of 20 levels 41.9 -> 40.1,
 // 14 336 of 75 139.6 -> 125.6, 30 240 155.2 -> 134.1, 53 760 161.7 -> 154.0,
 // 120 960 214.2 -> 200.0, 336 000 of 60 389.4 -> 363.1 (with 64 threads there
-// 376.0).  An ensemble's persistent launch wants no more than eight levels
-// (six members, 65 965 columns: 148.0 -> 131.8; 152.7 with 16).
+// 376.0).  An ensemble's persistent launch wants no more than eight levels:
+// us a step with 256 threads and none in LDS, this rule (eight at most), 64
+// threads and 16 levels -- 4 members, 27 000 columns x 40, two passives 86, 76,
+// 75; 6 unlike, 49 845 x 30 to 75 167, 152, 145; 16, 110 592 x 30 92, 81, 86; 8,
+// 144 000 x 50 159, 152, 169; 4, 518 400 x 75 750, 707, 889.
 void default_shape(rdb_colphys* h, long long columns, int nz, int max_levels) {
   if (h->block_pinned) return;
   int dev = 0, n_cu = 0;
