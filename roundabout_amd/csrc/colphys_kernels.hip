@@ -551,7 +551,7 @@ __global__ void k_first_live(StateView s, int p0, int p1) {
 }
 
 // The interfaces are independent: a lane takes PREP_LEVELS of one column's.
-// 480 x 360 x 75: 78 us, 4.7 TB/s (177 us when a lane walked its whole
+// 480 x 360 x 75: 78 us (177 us when a lane walked its whole
 // column, a memory round trip a level).  Needs s.kb.
 __global__ void k_prepare(StateView s, Params pr, int p0, int p1) {
   const int p = p0 + blockIdx.x * blockDim.x + threadIdx.x;

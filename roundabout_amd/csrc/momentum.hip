@@ -142,9 +142,9 @@ constexpr int MTPB = 128;
 // when it is done with level k waits a memory round trip a level: the levels
 // come through MPF register slots, loops unrolled by MPF so that every slot
 // index is a constant, and a load past the column's end re-reads its last
-// level, unused.  480 x 360 x 75, both directions: 554 -> 353 us, 5.2 TB/s
-// with the Thomas state (c' and d', 32 B a level out and back), which bounds
-// it now.
+// level, unused.  480 x 360 x 75, both directions: 554 -> 316 us.  What bounds
+// it now is HBM with the Thomas state (c' out and back, d' out and back in the
+// velocities): 1440 x 1080 x 75, 17.3 GB by the counters in 3.04 ms, 5.7 TB/s.
 // PLAIN: no option but the implicit wind stress (the flags' branches cost
 // registers and issue slots in every level); otherwise the flags decide.
 template <bool PLAIN>

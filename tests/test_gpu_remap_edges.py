@@ -84,7 +84,7 @@ def _far_targets(ho, hn, rng):
 @pytest.mark.parametrize("method", [1, 2, 3, 4, 5])
 def test_in_place_and_split_walks(orc, nx, ny, nz, method):
     """Below 65 537 columns a column's targets are split over lanes, above one
-    lane walks them, in place without a buffer: both, in place and out of
+    lane walks them, with scratch for what runs ahead: both, in place and out of
     place, on targets ahead of and behind their sources."""
     rng = np.random.default_rng(nz)
     ho, hn, c = _field(31, 20, nz, 90 + nz)
