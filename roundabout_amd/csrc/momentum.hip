@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(MTPB) k_vdiff_momentum(MomView vu, MomView vv,
   }
   const double d_min = mmin(-zcol_l, -zcol_r);
   int kb_live = kb;
-  for (int k = kb; k < nz; ++k) {
+  for (int k = fl.zlevel ? max(kb, 0) : kb; k < nz; ++k) {
     const bool live = fl.zlevel ? (mmin(v.h[cl + C * k], v.h[cr + C * k]) > HV) : true;
     if (live) {
       kb_live = k;
@@ -223,7 +223,8 @@ __global__ void __launch_bounds__(MTPB) k_vdiff_momentum(MomView vu, MomView vv,
   }
   // first row of the solve that is not the identity (a top row below the
   // first live one takes the top forcing: then every row is solved)
-  const int k_lo = (ktop < kb_live) ? 0 : kb_live;
+  // (k_bot below 1 leaves kb_live below the column: its rows start at 0)
+  const int k_lo = (ktop < kb_live) ? 0 : max(kb_live, 0);
   auto load = [&](int k, MomLevel& q) {
     const int kk = min(k, nz - 1);
     q.hl = v.h[cl + C * kk];

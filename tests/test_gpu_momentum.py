@@ -202,3 +202,32 @@ def test_work_arrays_of_a_solve():
         cp.synchronize()
         field = 8 * nz * (nx + 1) * ny
         assert before - free() < 6 * field + (32 << 20)
+
+
+@pytest.mark.parametrize("zlevel", [False, True])
+def test_bottom_rows_below_the_column(orc, zlevel):
+    """Faces whose k_bot is below 1, among ordinary ones: every row of theirs
+    is solved, and nothing outside the column is touched (the neighbouring
+    allocations' fields come back as they were set)."""
+    nx, ny, nz = 33, 18, 6
+    print(f"[case] momentum, k_bot below 1, {nx}x{ny}x{nz} zlevel={zlevel}", flush=True)
+    ocean = synth.make_ocean(nx, ny, nz, 8, land_frac=0.2, topo="zstar")
+    rng = np.random.default_rng(nz)
+    f = {}
+    for tag, shp in (("u", (nx + 1, ny)), ("v", (nx, ny + 1))):
+        f[f"k_bot_{tag}"] = np.where(rng.random(shp) < 0.5, 1 - rng.integers(1, 40, shp), 1).astype(float)
+        f[f"lambda_bot_{tag}"] = rng.uniform(0.0, 2e-4, shp)
+    kw = dict(implicit_stress=True, remnant=True, K_v_momentum=1e-2)
+    u, v, ru, rv = orc.vdiff_apply_momentum(ocean.h, ocean.u, ocean.v, ocean.wet, DT, tau_u=ocean.tau_x,
+                                            tau_v=ocean.tau_y, rho0=default_config().rho0, **f, **kw)
+    with ColumnPhysics.from_ocean(ocean) as cp:
+        for name, arr in f.items():
+            cp.set_field(name, arr)
+        cp.vdiff_momentum(DT, use_kv_source=0, implicit_stress=1, remnant=1, K_v_momentum=1e-2, zlevel_faces=int(zlevel))
+        for name, want in (("u_face_x_layer", u), ("v_face_y_layer", v), ("visc_rem_u", ru), ("visc_rem_v", rv)):
+            got = cp.get_field(name)
+            assert np.isfinite(got).all() if zlevel else np.array_equal(got, want), name
+        for name in ("temperature", "salinity", "h_layer"):
+            assert np.array_equal(cp.get_field(name), {"temperature": ocean.T, "salinity": ocean.S, "h_layer": ocean.h}[name])
+        for name, arr in f.items():
+            assert np.array_equal(np.asarray(cp.get_field(name)).reshape(arr.shape, order="F"), arr)
